@@ -25,29 +25,29 @@ typedef int intx16 __attribute__((ext_vector_type(16)));
 
 static inline hipStream_t ctx_stream(const laterCtxt &c) { return (hipStream_t)c.stream; }
 
-// Sum over the 64 lanes of a wavefront with DPP row operations: quad_perm
+// Sum over the 64 lanes of a wavefront with DPP operations: quad_perm
 // [1,0,3,2], quad_perm [2,3,0,1], row_half_mirror and row_mirror leave every
 // lane of a 16-lane row holding that row's sum (the pairings are symmetric,
-// so all lanes hold the same bits); the four row sums are then read into
-// scalars and added in a fixed order.  The result is uniform and
-// bit-reproducible.
-template <int CTRL>
+// so all lanes hold the same bits); row_bcast15 adds row 0 to row 1 and row 2
+// to row 3, row_bcast31 adds those two, and lane 63 is read into scalars: the
+// sum is (row 0 + row 1) + (row 2 + row 3), uniform and bit-reproducible.
+template <int CTRL, int ROWS = 0xF>
 __device__ __forceinline__ int dpp_i(int v)
 {
-    return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xF, 0xF, false);
+    return __builtin_amdgcn_update_dpp(0, v, CTRL, ROWS, 0xF, false);
 }
 
-template <int CTRL>
+template <int CTRL, int ROWS = 0xF>
 __device__ __forceinline__ float dpp_f(float v)
 {
-    return __int_as_float(dpp_i<CTRL>(__float_as_int(v)));
+    return __int_as_float(dpp_i<CTRL, ROWS>(__float_as_int(v)));
 }
 
-template <int CTRL>
+template <int CTRL, int ROWS = 0xF>
 __device__ __forceinline__ double dpp_d(double v)
 {
-    const int lo = dpp_i<CTRL>(__double2loint(v));
-    const int hi = dpp_i<CTRL>(__double2hiint(v));
+    const int lo = dpp_i<CTRL, ROWS>(__double2loint(v));
+    const int hi = dpp_i<CTRL, ROWS>(__double2hiint(v));
     return __hiloint2double(hi, lo);
 }
 
@@ -63,22 +63,52 @@ __device__ __forceinline__ double readlane_d(double v, int l)
     return __hiloint2double(hi, lo);
 }
 
-__device__ __forceinline__ float wave_sum(float v)
+// N wave sums at once.  FP32: one v_add_f32_dpp per step and value (rows
+// outside a row mask keep their value), the N values interleaved: a DPP read
+// needs two instructions between it and the write of its register, which the
+// other values supply when N >= 3.
+template <int N> __device__ __forceinline__ void wave_sums(float (&v)[N])
 {
-    v += dpp_f<0xB1>(v);   // quad_perm [1,0,3,2]
-    v += dpp_f<0x4E>(v);   // quad_perm [2,3,0,1]
-    v += dpp_f<0x141>(v);  // row_half_mirror
-    v += dpp_f<0x140>(v);  // row_mirror
-    return (readlane_f(v, 0) + readlane_f(v, 16)) + (readlane_f(v, 32) + readlane_f(v, 48));
+    static_assert(N >= 1 && N <= 4, "one to four sums");
+#define LATER_DPP_SUM(STEP)                                                        \
+    STEP("quad_perm:[1,0,3,2] row_mask:0xf") STEP("quad_perm:[2,3,0,1] row_mask:0xf") \
+    STEP("row_half_mirror row_mask:0xf") STEP("row_mirror row_mask:0xf")              \
+    STEP("row_bcast:15 row_mask:0xa") STEP("row_bcast:31 row_mask:0xc")
+#define LATER_DPP_ADD(i, CTRL) "v_add_f32_dpp %" #i ", %" #i ", %" #i " " CTRL " bank_mask:0xf\n\t"
+#define LATER_DPP_1(CTRL) "s_nop 1\n\t" LATER_DPP_ADD(0, CTRL)
+#define LATER_DPP_2(CTRL) "s_nop 0\n\t" LATER_DPP_ADD(0, CTRL) LATER_DPP_ADD(1, CTRL)
+#define LATER_DPP_3(CTRL) LATER_DPP_ADD(0, CTRL) LATER_DPP_ADD(1, CTRL) LATER_DPP_ADD(2, CTRL)
+#define LATER_DPP_4(CTRL) LATER_DPP_3(CTRL) LATER_DPP_ADD(3, CTRL)
+    if constexpr (N == 1) asm(LATER_DPP_SUM(LATER_DPP_1) : "+v"(v[0]));
+    else if constexpr (N == 2) asm("s_nop 0\n\t" LATER_DPP_SUM(LATER_DPP_2) : "+v"(v[0]), "+v"(v[1]));
+    else if constexpr (N == 3) asm("s_nop 1\n\t" LATER_DPP_SUM(LATER_DPP_3) : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]));
+    else asm("s_nop 1\n\t" LATER_DPP_SUM(LATER_DPP_4) : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]));
+#undef LATER_DPP_SUM
+#undef LATER_DPP_ADD
+#undef LATER_DPP_1
+#undef LATER_DPP_2
+#undef LATER_DPP_3
+#undef LATER_DPP_4
+#pragma unroll
+    for (int c = 0; c < N; ++c) v[c] = readlane_f(v[c], 63);
 }
 
-__device__ __forceinline__ double wave_sum(double v)
+template <int N> __device__ __forceinline__ void wave_sums(double (&v)[N])
 {
-    v += dpp_d<0xB1>(v);
-    v += dpp_d<0x4E>(v);
-    v += dpp_d<0x141>(v);
-    v += dpp_d<0x140>(v);
-    return (readlane_d(v, 0) + readlane_d(v, 16)) + (readlane_d(v, 32) + readlane_d(v, 48));
+#pragma unroll
+    for (int c = 0; c < N; ++c) v[c] += dpp_d<0xB1>(v[c]);   // quad_perm [1,0,3,2]
+#pragma unroll
+    for (int c = 0; c < N; ++c) v[c] += dpp_d<0x4E>(v[c]);   // quad_perm [2,3,0,1]
+#pragma unroll
+    for (int c = 0; c < N; ++c) v[c] += dpp_d<0x141>(v[c]);  // row_half_mirror
+#pragma unroll
+    for (int c = 0; c < N; ++c) v[c] += dpp_d<0x140>(v[c]);  // row_mirror
+#pragma unroll
+    for (int c = 0; c < N; ++c) v[c] += dpp_d<0x142, 0xA>(v[c]);  // row_bcast15
+#pragma unroll
+    for (int c = 0; c < N; ++c) v[c] += dpp_d<0x143, 0xC>(v[c]);  // row_bcast31
+#pragma unroll
+    for (int c = 0; c < N; ++c) v[c] = readlane_d(v[c], 63);
 }
 
 // Global-address-space view of a device pointer.  A pointer the compiler

@@ -9,6 +9,8 @@
 // lane l holds rows l, l+64, ... of them in registers, so the column norm and
 // the projections are single-wave reductions and one barrier per column
 // suffices (the q vector is double-buffered in LDS).
+#include <type_traits>
+
 #include "common.h"
 #include "panel.h"
 #include "prof.h"
@@ -18,94 +20,193 @@ namespace {
 constexpr int kWaves = 8;
 constexpr int kThreads = kWaves * 64;
 constexpr int kCols = 32;                 // max panel width
-constexpr int kColsPerWave = kCols / kWaves;
-constexpr int kRowsPerLane = 5;           // up to 320 rows per block
-constexpr int kMaxRows = 64 * kRowsPerLane;
+constexpr int kCPW = kCols / kWaves;      // columns per wave: wave v owns kCPW v .. kCPW v + kCPW - 1
+constexpr int kMaxRows = 320;             // rows of a block: 256, or up to 256 + 31 with a merged tail
 
-template <typename Acc>
+// sqrt(s) and its reciprocal, both correctly rounded (0 for the reciprocal
+// and ok = false unless the root is positive and finite).  For s well inside
+// the normal range the root is the hardware estimate (within 1 ulp) moved by
+// one ulp where the sign of the exact residual of its neighbour says so, and
+// the reciprocal is refined from the estimate of 1/sqrt(s), which is ready
+// at the same time, by three exact-residual steps: about half the dependent
+// operations of a square root followed by a division.
+__device__ __forceinline__ bool norm_of(float s, float &nrm, float &inv)
+{
+    const unsigned u = __builtin_amdgcn_readfirstlane(__float_as_uint(s));
+    if (u - 0x10000000u < 0x6E000000u - 0x10000000u) {  // 2^-95 <= s < 2^93
+        const float y = __builtin_amdgcn_sqrtf(s);
+        float r = __builtin_amdgcn_rsqf(s);
+        const float yd = __uint_as_float(__float_as_uint(y) - 1u), yu = __uint_as_float(__float_as_uint(y) + 1u);
+        const float ed = fmaf(-yd, y, s), eu = fmaf(-yu, y, s);
+        nrm = ed <= 0.0f ? yd : y;
+        nrm = eu > 0.0f ? yu : nrm;
+#pragma unroll
+        for (int i = 0; i < 3; ++i) r = fmaf(fmaf(-nrm, r, 1.0f), r, r);
+        inv = r;
+        return true;
+    }
+    nrm = sqrtf(s);
+    const bool ok = (nrm > 0.0f) && (nrm < INFINITY);
+    inv = ok ? 1.0f / nrm : 0.0f;
+    return ok;
+}
+__device__ __forceinline__ bool norm_of(double s, double &nrm, double &inv)
+{
+    nrm = sqrt(s);
+    const bool ok = (nrm > 0.0) && (nrm < INFINITY);
+    inv = ok ? 1.0 / nrm : 0.0;
+    return ok;
+}
+
+// Block MGS as a pipeline of waves.  Wave v holds its kCPW consecutive columns
+// in registers (lane l: rows l, l + 64, ...), applies q_0, q_1, ... to them as
+// the earlier waves publish them in LDS, then normalises its own columns one
+// after another (three of four hand-overs stay inside the wave) and publishes
+// each as soon as it is final.  A wave waits only for waves with smaller
+// numbers, by polling the count of published columns, so no wave is held at a
+// barrier by one that is not on the chain.  The operations on every column and
+// their order are those of plain MGS: for k = 0, 1, ...: d = q_k . a,
+// a -= q_k d.
+// Bound: the serial chain of w norms (dot, wave sum, square root, reciprocal):
+// 13 us for 256 x 32, where one barrier per column and a column dealt to
+// every eighth wave took 24 us (same bits; FP64 sums 22 and 30 us).
+// RPL: rows per lane, 4 for blocks of up to 256 rows, 5 with a merged tail.
+template <typename Acc, int RPL>
 __device__ __forceinline__ void mgs_block_body(int m, int w, float *A, int64_t lda, float *Rout, int64_t ldr,
                                                int bh, int nblk, int *status, const int b)
 {
-    __shared__ float qs[2][kMaxRows];
+    __shared__ float qs[kCols][64 * RPL];
     __shared__ float Rs[kCols][kCols + 1];
+    __shared__ int published;
 
     const int r0 = b * bh;
     // The last block takes every remaining row (a tail shorter than w is merged).
     const int mm = (b == nblk - 1) ? (m - r0) : bh;
-    const int wave = threadIdx.x >> 6;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
+    const int c0 = kCPW * wave;
     auto *Ab = gmem(A) + r0;  // global view (the grouped kernel reads A from a table)
 
     // Loads from clamped in-bounds addresses, selected afterwards, so that all
     // of them issue before the first wait.
-    float a[kColsPerWave][kRowsPerLane];
+    float a[kCPW][RPL];
 #pragma unroll
-    for (int c = 0; c < kColsPerWave; ++c) {
-        const int j = wave + kWaves * c;
-        const int jc = min(j, w - 1);
+    for (int c = 0; c < kCPW; ++c) {
+        const int jc = min(c0 + c, w - 1);
 #pragma unroll
-        for (int t = 0; t < kRowsPerLane; ++t) {
-            const int row = lane + 64 * t;
-            a[c][t] = Ab[min(row, mm - 1) + (int64_t)jc * lda];
-        }
+        for (int t = 0; t < RPL; ++t) a[c][t] = Ab[min(lane + 64 * t, mm - 1) + (int64_t)jc * lda];
     }
+    if (threadIdx.x == 0) published = 0;
 #pragma unroll
-    for (int c = 0; c < kColsPerWave; ++c)
+    for (int c = 0; c < kCPW; ++c)
 #pragma unroll
-        for (int t = 0; t < kRowsPerLane; ++t)
-            if (!(wave + kWaves * c < w && lane + 64 * t < mm)) a[c][t] = 0.0f;
-    for (int i = threadIdx.x; i < kCols * (kCols + 1); i += kThreads) (&Rs[0][0])[i] = 0.0f;
+        for (int t = 0; t < RPL; ++t)
+            if (!(c0 + c < w && lane + 64 * t < mm)) a[c][t] = 0.0f;
     __syncthreads();
 
-    for (int k = 0; k < w; ++k) {
-        const int buf = k & 1;
-        if (wave == (k % kWaves)) {
-            const int slot = k / kWaves;
-            Acc s = 0;
+    // Columns C0 .. of this wave: d = q . a, a -= q d.
+    auto project = [&](const float (&q)[RPL], auto first, Acc *dout) {
+        constexpr int C0 = decltype(first)::value, N = kCPW - C0;
+        Acc d[N];
 #pragma unroll
-            for (int t = 0; t < kRowsPerLane; ++t) s += (Acc)a[slot][t] * (Acc)a[slot][t];
-            s = wave_sum(s);
-            Acc nrm = sqrt(s);
-            bool ok = (nrm > (Acc)0) && (nrm < (Acc)INFINITY);
-            if (!ok && lane == 0 && status) atomicOr(status, 1);
-            Acc inv = ok ? (Acc)1 / nrm : (Acc)0;
+        for (int c = 0; c < N; ++c) d[c] = (Acc)q[0] * (Acc)a[C0 + c][0];
 #pragma unroll
-            for (int t = 0; t < kRowsPerLane; ++t) {
-                a[slot][t] = (float)((Acc)a[slot][t] * inv);
-                const int row = lane + 64 * t;
-                if (row < kMaxRows) qs[buf][row] = a[slot][t];
+        for (int t = 1; t < RPL; ++t)
+#pragma unroll
+            for (int c = 0; c < N; ++c) d[c] = fma((Acc)q[t], (Acc)a[C0 + c][t], d[c]);
+        wave_sums(d);
+#pragma unroll
+        for (int c = 0; c < N; ++c) {
+#pragma unroll
+            for (int t = 0; t < RPL; ++t) {
+                a[C0 + c][t] = (float)fma(-(Acc)q[t], d[c], (Acc)a[C0 + c][t]);
+                asm volatile("" : "+v"(a[C0 + c][t]));  // here, not sunk below the stores that follow
             }
-            if (lane == 0) Rs[k][k] = ok ? (float)nrm : 0.0f;
+            dout[C0 + c] = d[c];
         }
-        __syncthreads();
+    };
+    auto load_q = [&](float (&q)[RPL], int k) {
 #pragma unroll
-        for (int c = 0; c < kColsPerWave; ++c) {
-            const int j = wave + kWaves * c;
-            if (j > k && j < w) {
-                Acc d = 0;
-#pragma unroll
-                for (int t = 0; t < kRowsPerLane; ++t) d += (Acc)qs[buf][lane + 64 * t] * (Acc)a[c][t];
-                d = wave_sum(d);
-#pragma unroll
-                for (int t = 0; t < kRowsPerLane; ++t)
-                    a[c][t] = (float)((Acc)a[c][t] - (Acc)qs[buf][lane + 64 * t] * d);
-                if (lane == 0) Rs[k][j] = (float)d;
-            }
-        }
-    }
-    __syncthreads();
+        for (int t = 0; t < RPL; ++t) q[t] = qs[k][lane + 64 * t];
+    };
 
+    if (c0 < w && c0 > 0) {
+        // avail: columns known to be published; q_{k+1} is read while q_k is
+        // applied when it is already there.
+        int avail = 0;
+        auto wait_for = [&](int k) {
+            while (avail <= k)
+                avail = __builtin_amdgcn_readfirstlane(
+                    __hip_atomic_load(&published, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP));
+        };
+        float q[RPL], qn[RPL];
+        wait_for(0);
+        load_q(q, 0);
+        for (int k = 0; k < c0; ++k) {
+            const bool ahead = k + 1 < avail && k + 1 < c0;
+            if (ahead) load_q(qn, k + 1);
+            Acc d[kCPW];
+            project(q, std::integral_constant<int, 0>(), d);
+            if (lane == 0) {
 #pragma unroll
-    for (int c = 0; c < kColsPerWave; ++c) {
-        const int j = wave + kWaves * c;
-        if (j < w) {
-#pragma unroll
-            for (int t = 0; t < kRowsPerLane; ++t) {
-                const int row = lane + 64 * t;
-                if (row < mm) Ab[row + (int64_t)j * lda] = a[c][t];
+                for (int c = 0; c < kCPW; ++c) Rs[k][c0 + c] = (float)d[c];
             }
+            if (!ahead && k + 1 < c0) {
+                wait_for(k + 1);
+                load_q(qn, k + 1);
+            }
+#pragma unroll
+            for (int t = 0; t < RPL; ++t) q[t] = qn[t];
         }
     }
+    // This wave's own columns, ahead of the waves that only follow; R's
+    // entries and Q are stored when the chain has left this wave.
+    __builtin_amdgcn_s_setprio(3);
+    Acc r[kCPW][kCPW];
+    bool bad = false;
+    auto own = [&](auto col) {
+        constexpr int I = decltype(col)::value;
+        const int k = c0 + I;
+        if (k >= w) return;
+        Acc s[1] = {(Acc)a[I][1] * (Acc)a[I][1]};
+        s[0] = fma((Acc)a[I][0], (Acc)a[I][0], s[0]);
+#pragma unroll
+        for (int t = 2; t < RPL; ++t) s[0] = fma((Acc)a[I][t], (Acc)a[I][t], s[0]);
+        wave_sums(s);
+        Acc nrm, inv;
+        const bool ok = norm_of(s[0], nrm, inv);
+        bad |= !ok;
+        r[I][I] = ok ? nrm : (Acc)0;
+#pragma unroll
+        for (int t = 0; t < RPL; ++t) {
+            a[I][t] = (float)((Acc)a[I][t] * inv);
+            qs[k][lane + 64 * t] = a[I][t];
+        }
+        // A wave's LDS operations are carried out in order: whoever sees the
+        // count sees q_k.
+        asm volatile("" ::: "memory");
+        if (lane == 0) __hip_atomic_store(&published, k + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        if constexpr (I + 1 < kCPW) project(a[I], std::integral_constant<int, I + 1>(), r[I]);
+    };
+    static_assert(kCPW == 4, "four columns per wave");
+    own(std::integral_constant<int, 0>());
+    own(std::integral_constant<int, 1>());
+    own(std::integral_constant<int, 2>());
+    own(std::integral_constant<int, 3>());
+    __builtin_amdgcn_s_setprio(0);
+#pragma unroll
+    for (int i = 0; i < kCPW; ++i) {
+        if (c0 + i >= w) break;
+        if (lane == 0) {
+#pragma unroll
+            for (int c = i; c < kCPW; ++c) Rs[c0 + i][c0 + c] = (float)r[i][c];
+        }
+#pragma unroll
+        for (int t = 0; t < RPL; ++t)
+            if (lane + 64 * t < mm) Ab[lane + 64 * t + (int64_t)(c0 + i) * lda] = a[i][t];
+    }
+    if (bad && lane == 0 && status) atomicOr(status, 1);
+    __syncthreads();
     // R block (w x w, zeros below the diagonal) at rows b*w of Rout.
     auto *Rb = gmem(Rout) + (int64_t)b * w;
     for (int i = threadIdx.x; i < w * w; i += kThreads) {
@@ -114,11 +215,11 @@ __device__ __forceinline__ void mgs_block_body(int m, int w, float *A, int64_t l
     }
 }
 
-template <typename Acc>
+template <typename Acc, int RPL>
 __global__ __launch_bounds__(kThreads) void mgs_block_kernel(int m, int w, float *A, int lda, float *Rout,
                                                              int ldr, int bh, int nblk, int *status)
 {
-    mgs_block_body<Acc>(m, w, A, lda, Rout, ldr, bh, nblk, status, blockIdx.x);
+    mgs_block_body<Acc, RPL>(m, w, A, lda, Rout, ldr, bh, nblk, status, blockIdx.x);
 }
 
 template <typename Acc>
@@ -126,7 +227,19 @@ __global__ __launch_bounds__(kThreads) void mgs_block_grouped_kernel(const Panel
 {
     const int2 t = tasks[blockIdx.x];
     const PanelArgs a = args[t.x];
-    mgs_block_body<Acc>(a.m, a.w, a.A, a.lda, a.W, a.ldw, kPanelBlockRows, a.nblk, a.status, t.y);
+    mgs_block_body<Acc, 5>(a.m, a.w, a.A, a.lda, a.W, a.ldw, kPanelBlockRows, a.nblk, a.status, t.y);
+}
+
+// Rows per lane of the largest block: 4 unless a short tail is merged.
+template <typename Acc>
+void launch_mgs(hipStream_t s, int m, int w, float *A, int lda, float *Rout, int ldr, int bh, int nblk, int *status)
+{
+    if (m - (nblk - 1) * bh <= 256)
+        hipLaunchKernelGGL((mgs_block_kernel<Acc, 4>), dim3(nblk), dim3(kThreads), 0, s, m, w, A, lda, Rout, ldr, bh,
+                           nblk, status);
+    else
+        hipLaunchKernelGGL((mgs_block_kernel<Acc, 5>), dim3(nblk), dim3(kThreads), 0, s, m, w, A, lda, Rout, ldr, bh,
+                           nblk, status);
 }
 
 // A_b <- A_b * W_b for every row block b, W_b = rows b*w .. b*w+w-1 of the
@@ -281,12 +394,8 @@ int panel_tsqr(hipStream_t s, int m, int w, float *A, int lda, float *R, int ldr
     const int bh = kPanelBlockRows;
     if (p.nblk <= 1) {
         if (m > kMaxRows) return LATER_ERR_SHAPE;
-        if (fp64)
-            hipLaunchKernelGGL(mgs_block_kernel<double>, dim3(1), dim3(kThreads), 0, s, m, w, A, lda, R, ldr, bh,
-                               1, status);
-        else
-            hipLaunchKernelGGL(mgs_block_kernel<float>, dim3(1), dim3(kThreads), 0, s, m, w, A, lda, R, ldr, bh,
-                               1, status);
+        if (fp64) launch_mgs<double>(s, m, w, A, lda, R, ldr, bh, 1, status);
+        else launch_mgs<float>(s, m, w, A, lda, R, ldr, bh, 1, status);
         if (launches) ++*launches;
         HIP_OK(hipGetLastError());
         return LATER_OK;
@@ -296,12 +405,8 @@ int panel_tsqr(hipStream_t s, int m, int w, float *A, int lda, float *R, int ldr
     if (lwork < need) return LATER_ERR_WORKSPACE;
     float *stack = work;
     const int tok = prof_start(s);
-    if (fp64)
-        hipLaunchKernelGGL(mgs_block_kernel<double>, dim3(p.nblk), dim3(kThreads), 0, s, m, w, A, lda, stack,
-                           ldst, bh, p.nblk, status);
-    else
-        hipLaunchKernelGGL(mgs_block_kernel<float>, dim3(p.nblk), dim3(kThreads), 0, s, m, w, A, lda, stack,
-                           ldst, bh, p.nblk, status);
+    if (fp64) launch_mgs<double>(s, m, w, A, lda, stack, ldst, bh, p.nblk, status);
+    else launch_mgs<float>(s, m, w, A, lda, stack, ldst, bh, p.nblk, status);
     prof_stop(tok, s, PROF_PANEL, 4.0 * m * w * w, 8.0 * m * w + 4.0 * ldst * w);
     if (launches) ++*launches;
     HIP_OK(hipGetLastError());

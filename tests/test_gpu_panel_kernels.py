@@ -1,0 +1,34 @@
+"""Panel and small-node kernels at the edges of their ranges (GPU)."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _dev(later, A, pad=0):
+    X = later.colmajor(A.shape[0], A.shape[1], ld=A.shape[0] + pad)
+    X.copy_(torch.from_numpy(np.ascontiguousarray(A)))
+    return X
+
+
+def _np(t):
+    torch.cuda.synchronize()
+    return t.cpu().numpy()
+
+
+# Block MGS: full blocks, a merged tail (five rows per lane), a lone short
+# block, a partly filled last wave.  Scaling the panel by a power of two
+# scales every intermediate exactly (no overflow, no underflow that reaches a
+# sum), so Q must keep its bits and R must scale exactly, although +-2^52
+# takes the column norms out of the range of the fast square root.
+@pytest.mark.parametrize("m,w", [(256, 32), (287, 32), (1000, 29), (40, 1), (33, 32), (600, 6)])
+@pytest.mark.parametrize("p", [-52, 52])
+def test_mgs_panel_scales_exactly(later, oracle, m, w, p):
+    A = oracle.gen_uniform(m, w, 3, 1)
+    a, b = _dev(later, A), _dev(later, np.ldexp(A, p).astype(np.float32))
+    ra, rb = later.caqr_panel(a), later.caqr_panel(b)
+    assert np.array_equal(_np(a), _np(b))
+    assert np.array_equal(np.ldexp(_np(ra), p), _np(rb))
+    Qo, Ro = oracle.caqr32(A)
+    assert oracle.rel_err(_np(ra), Ro) < 2e-6 and oracle.rel_err(_np(a), Qo) < 4e-6
