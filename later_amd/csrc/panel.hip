@@ -287,42 +287,146 @@ __global__ __launch_bounds__(256) void tsqr_apply_grouped_kernel(const PanelArgs
     tsqr_apply_body<Acc>(a.m, a.w, a.A, a.lda, a.W, a.ldw, kPanelBlockRows, a.nblk, t.y);
 }
 
-// The same product over 64-row tiles of the panel (four waves per tile: the
-// tile is staged in LDS, wave q forms output columns q, q+4, ...), so that a
-// 16384-row panel spreads over 256 workgroups instead of 64.  Every output
-// keeps the row-per-thread form's order of summation over k, so the two give
-// the same bits.  A tile never straddles two 256-row blocks; the tiles of a
-// merged tail belong to the last block.
-constexpr int kApplyRows = 64;
-
-template <typename Acc>
-__global__ __launch_bounds__(256) void tsqr_apply_tile_kernel(int m, int w, float *A, int lda, const float *W,
-                                                              int ldw, int bh, int nblk)
+// The same product for a panel of its own launch, in the same order of
+// summation over k (the same bits).  Two layouts: CG = 4 gives a workgroup 64
+// rows, each wave a quarter of the output columns (a 16384-row panel then
+// covers the chip); CG = 1 gives it a whole 256-row block, each wave 64 rows
+// and every column (an eighth of the W traffic per row, no barrier between
+// reading and writing A: for panels with a block for every CU).
+// FUSED: W is itself still to be multiplied by its rows of the next level's
+// Q, W2 (blocks of 256 rows of W, W2's rows b2 w ..); the workgroup forms its
+// w x w product W_b W2_b2 first, rounded to FP32 as the separate launch would
+// store it, which saves that launch and a round trip of the stack.
+// W is kept k-contiguous in LDS and read as broadcast 16-byte vectors, all of
+// A's loads are in flight before the first wait: 16384 x 32 takes 7.1 us with
+// the next level's product in it and 4.9 us without, where two launches took
+// 14.5 us each with runtime-strided staging and scalar LDS reads.
+template <typename Acc, int CG, bool FUSED>
+__global__ __launch_bounds__(256) void tsqr_apply_kernel(int m, int w, float *A, int lda, const float *W, int ldw,
+                                                         int nblk, const float *W2, int ldw2, int nblk2)
 {
-    __shared__ float Ws[kCols][kCols];
-    __shared__ float Vs[kCols][kApplyRows];
-    const int row0 = blockIdx.x * kApplyRows;
-    const int b = min(row0 / bh, nblk - 1);
-    const int rows = min(kApplyRows, m - row0);
-    const auto *Wb = gmem(W) + (int64_t)b * w;
-    for (int i = threadIdx.x; i < w * w; i += 256) {
-        const int x = i % w, y = i / w;
-        Ws[x][y] = Wb[x + (int64_t)y * ldw];
-    }
-    const int r = threadIdx.x & 63, q = threadIdx.x >> 6;
-    float *At = A + row0;
-    for (int c = q; c < w; c += 4) Vs[c][r] = (r < rows) ? At[r + (int64_t)c * lda] : 0.0f;
-    __syncthreads();
+    constexpr int bh = kPanelBlockRows;
+    __shared__ __attribute__((aligned(16))) Acc Ws[kCols][kCols];  // [j][k]
+    __shared__ float S1[FUSED ? kCols : 1][kCols + 1], S2[FUSED ? 2 : 1][FUSED ? kCols : 1][kCols + 1];
+    const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int b = (CG == 4) ? min((int)blockIdx.x * 64 / bh, nblk - 1) : (int)blockIdx.x;
+    const int rend = (b == nblk - 1) ? m : (b + 1) * bh;  // rows of the block end here
+    const int row0 = (CG == 4) ? (int)blockIdx.x * 64 : b * bh + 64 * wv;
+
     float v[kCols];
+    auto load_rows = [&](int r0) {
+        const float *src = A + min(r0 + lane, rend - 1);
 #pragma unroll
-    for (int k = 0; k < kCols; ++k) v[k] = (k < w) ? Vs[k][r] : 0.0f;
-    for (int j = q; j < w; j += 4) {
-        Acc s = 0;
+        for (int k = 0; k < kCols; ++k) v[k] = src[(int64_t)min(k, w - 1) * lda];
+    };
+    if (CG == 4 || row0 < rend) load_rows(row0);
+
+    const int x = tid & 31;
+    if constexpr (!FUSED) {
 #pragma unroll
-        for (int k = 0; k < kCols; ++k)
-            if (k < w) s += (Acc)v[k] * (Acc)Ws[k][j];
-        if (r < rows) At[r + (int64_t)j * lda] = (float)s;
+        for (int u = 0; u < 4; ++u) {
+            const int y = (tid >> 5) + 8 * u;
+            const float t = W[(int64_t)b * w + min(x, w - 1) + (int64_t)min(y, w - 1) * ldw];
+            Ws[y][x] = (x < w && y < w) ? (Acc)t : (Acc)0;
+        }
+    } else {
+        // Rows g = b w + i of W lie in block min(g / 256, nblk2 - 1) of the
+        // next level: one block, or two where w does not divide 256.
+        const int b0 = min(b * w / bh, nblk2 - 1), b1 = min((b * w + w - 1) / bh, nblk2 - 1);
+        float t1[4], t2[4], t3[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int xc = min(x, w - 1), yc = min((tid >> 5) + 8 * u, w - 1);
+            t1[u] = W[(int64_t)b * w + xc + (int64_t)yc * ldw];
+            t2[u] = W2[(int64_t)b0 * w + xc + (int64_t)yc * ldw2];
+            t3[u] = W2[(int64_t)b1 * w + xc + (int64_t)yc * ldw2];
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int y = (tid >> 5) + 8 * u;
+            S1[x][y] = t1[u];
+            S2[0][x][y] = t2[u];
+            S2[1][x][y] = t3[u];
+        }
+        __syncthreads();
+        const int sel = (b * w + x) / bh > b0 && b1 > b0 ? 1 : 0;
+        Acc s[4] = {0, 0, 0, 0};
+        for (int k = 0; k < w; ++k) {
+            const Acc l = (Acc)S1[x][k];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) s[u] = fma(l, (Acc)S2[sel][k][(tid >> 5) + 8 * u], s[u]);
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int y = (tid >> 5) + 8 * u;
+            Ws[y][x] = (x < w && y < w) ? (Acc)(float)s[u] : (Acc)0;
+        }
     }
+#pragma unroll
+    for (int k = 0; k < kCols; ++k)
+        if (k >= w) v[k] = 0.0f;
+    // With CG = 4 this also orders every wave's reads of the tile before any
+    // wave's writes to it.
+    __syncthreads();
+
+    constexpr int NJ = 4, VW = 16 / sizeof(Acc);  // columns in flight, values of W per LDS read
+    typedef Acc vec_t __attribute__((ext_vector_type(VW)));
+    auto product = [&](int r0) {
+        const int row = r0 + lane;
+        const int jbeg = (CG == 4) ? 8 * wv : 0, jend = min(w, (CG == 4) ? 8 * wv + 8 : kCols);
+        for (int j = jbeg; j < jend; j += NJ) {
+            Acc s[NJ];
+#pragma unroll
+            for (int c = 0; c < NJ; ++c) s[c] = (Acc)0;
+#pragma unroll
+            for (int k = 0; k < kCols; k += VW) {
+                vec_t wk[NJ];
+#pragma unroll
+                for (int c = 0; c < NJ; ++c) wk[c] = *(const vec_t *)&Ws[j + c][k];
+#pragma unroll
+                for (int e = 0; e < VW; ++e)
+#pragma unroll
+                    for (int c = 0; c < NJ; ++c) s[c] = fma((Acc)v[k + e], wk[c][e], s[c]);
+            }
+            if (row < rend) {
+#pragma unroll
+                for (int c = 0; c < NJ; ++c)
+                    if (j + c < w) A[row + (int64_t)(j + c) * lda] = (float)s[c];
+            }
+        }
+    };
+    if constexpr (CG == 4) {
+        product(row0);
+    } else {
+        for (int r0 = row0; r0 < rend; r0 += 256) {  // a second round only for a merged tail
+            if (r0 != row0) {
+                load_rows(r0);
+#pragma unroll
+                for (int k = 0; k < kCols; ++k)
+                    if (k >= w) v[k] = 0.0f;
+            }
+            product(r0);
+        }
+    }
+}
+
+// A_b <- A_b W_b (W2 given: W_b W2_b2 in place of W_b) over the m x w panel.
+template <typename Acc>
+void launch_apply(hipStream_t s, int m, int w, float *A, int lda, const float *W, int ldw, int nblk, const float *W2,
+                  int ldw2, int nblk2)
+{
+    // A workgroup per block once that gives every CU one: below, the four
+    // times finer grid hides the latency of the loads (16384 rows: 7.1 us).
+    const bool whole = nblk >= 256;
+    const dim3 grid(whole ? nblk : (m + 63) / 64);
+#define LATER_APPLY(CG, F)                                                                                          \
+    hipLaunchKernelGGL((tsqr_apply_kernel<Acc, CG, F>), grid, dim3(256), 0, s, m, w, A, lda, W, ldw, nblk, W2, ldw2, \
+                       nblk2)
+    if (whole && W2) LATER_APPLY(1, true);
+    else if (whole) LATER_APPLY(1, false);
+    else if (W2) LATER_APPLY(4, true);
+    else LATER_APPLY(4, false);
+#undef LATER_APPLY
 }
 
 struct Blocks {
@@ -386,11 +490,18 @@ int64_t panel_work_floats(int m, int w)
     return tot;
 }
 
-int panel_tsqr(hipStream_t s, int m, int w, float *A, int lda, float *R, int ldr, float *work,
-               int64_t lwork, bool fp64, int *status, int *launches)
+namespace {
+
+// The MGS launches of the tree below an m x w panel; *stack, *ldst: its
+// level's stacked factors, whose Q rows the panel's blocks are multiplied by
+// (none when the panel is a single block).  apply_here: multiply the panel
+// too; otherwise the caller folds that product into its own.
+int tsqr_level(hipStream_t s, int m, int w, float *A, int lda, float *R, int ldr, float *work, int64_t lwork,
+               bool fp64, int *status, int *launches, bool apply_here, const float **stack_out, int *ldst_out)
 {
-    if (w < 1 || w > kCols || m < w) return LATER_ERR_SHAPE;
-    Blocks p = plan_blocks(m, w);
+    *stack_out = nullptr;
+    *ldst_out = 0;
+    const Blocks p = plan_blocks(m, w);
     const int bh = kPanelBlockRows;
     if (p.nblk <= 1) {
         if (m > kMaxRows) return LATER_ERR_SHAPE;
@@ -410,16 +521,30 @@ int panel_tsqr(hipStream_t s, int m, int w, float *A, int lda, float *R, int ldr
     prof_stop(tok, s, PROF_PANEL, 4.0 * m * w * w, 8.0 * m * w + 4.0 * ldst * w);
     if (launches) ++*launches;
     HIP_OK(hipGetLastError());
-    int rc = panel_tsqr(s, ldst, w, stack, ldst, R, ldr, work + need, lwork - need, fp64, status, launches);
+    // Levels are applied in pairs: this one's product takes the next one's in.
+    const float *stack2 = nullptr;
+    int ldst2 = 0;
+    const int rc = tsqr_level(s, ldst, w, stack, ldst, R, ldr, work + need, lwork - need, fp64, status, launches,
+                              !apply_here, &stack2, &ldst2);
     if (rc) return rc;
-    const int tiles = (m + kApplyRows - 1) / kApplyRows;
-    if (fp64)
-        hipLaunchKernelGGL(tsqr_apply_tile_kernel<double>, dim3(tiles), dim3(256), 0, s, m, w, A, lda, stack, ldst,
-                           bh, p.nblk);
-    else
-        hipLaunchKernelGGL(tsqr_apply_tile_kernel<float>, dim3(tiles), dim3(256), 0, s, m, w, A, lda, stack, ldst,
-                           bh, p.nblk);
+    *stack_out = stack;
+    *ldst_out = ldst;
+    if (!apply_here) return LATER_OK;
+    const int nblk2 = plan_blocks(ldst, w).nblk;
+    if (fp64) launch_apply<double>(s, m, w, A, lda, stack, ldst, p.nblk, stack2, ldst2, nblk2);
+    else launch_apply<float>(s, m, w, A, lda, stack, ldst, p.nblk, stack2, ldst2, nblk2);
     if (launches) ++*launches;
     HIP_OK(hipGetLastError());
     return LATER_OK;
+}
+
+} // namespace
+
+int panel_tsqr(hipStream_t s, int m, int w, float *A, int lda, float *R, int ldr, float *work,
+               int64_t lwork, bool fp64, int *status, int *launches)
+{
+    if (w < 1 || w > kCols || m < w) return LATER_ERR_SHAPE;
+    const float *stack;
+    int ldst;
+    return tsqr_level(s, m, w, A, lda, R, ldr, work, lwork, fp64, status, launches, true, &stack, &ldst);
 }

@@ -32,3 +32,19 @@ def test_mgs_panel_scales_exactly(later, oracle, m, w, p):
     assert np.array_equal(np.ldexp(_np(ra), p), _np(rb))
     Qo, Ro = oracle.caqr32(A)
     assert oracle.rel_err(_np(ra), Ro) < 2e-6 and oracle.rel_err(_np(a), Qo) < 4e-6
+
+
+# Tree apply: the next level's product folded in (two levels), a level left to
+# its own launch (three), w that does not divide 256 (rows of one stack block
+# in two blocks of the next level), a workgroup per block (256 blocks and
+# more) with a merged tail.
+@pytest.mark.parametrize("m,w", [(520, 20), (5000, 20), (9000, 31), (65536 + 9, 20), (70003, 29), (132000, 32)])
+@pytest.mark.parametrize("fp64", [0, 1])
+def test_tsqr_apply_levels(later, oracle, m, w, fp64):
+    A = oracle.gen_uniform(m, w, 5, 2)
+    X = _dev(later, A, pad=1)
+    R = later.caqr_panel(X, fp64=fp64)
+    Q, R = _np(X), _np(R)
+    Qo, Ro = oracle.caqr32(A)
+    assert oracle.rel_err(R, Ro) < 2e-6 and oracle.rel_err(Q, Qo) < 4e-6
+    assert oracle.orth(Q) < (2e-6 if fp64 else 4e-6) * np.sqrt(w)
