@@ -3,6 +3,8 @@
 // (panel_chol.hip) and the one-workgroup-per-matrix batched kernel
 // (batch_wg.hip).
 #pragma once
+#include <type_traits>
+
 #include "common.h"
 
 namespace {
@@ -197,136 +199,200 @@ __device__ __forceinline__ double readlane_f64(double v, int lane)
     return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
 }
 
-// Cholesky S = R^T R of a 32 x 32 block in LDS by one wave, and R^{-1}, in
-// one right-looking elimination, fully unrolled.  Lane j < 32 keeps column j
-// of the trailing matrix in registers; lane 32 + c keeps column c of the
-// identity, to which the same row operations are applied (Gauss-Jordan on
-// [S | I]): it ends as column c of the unit-lower M with M S = D L^T, and
-// R^{-1}[c][k] = M[k][c] / sqrt(d_k).  Column k's multipliers S[i][k] are read
-// from lane k with v_readlane and serve both halves.
-// S: row stride LDS_; d0[k]: the squared norm of column k that the pivot is
-// compared with; R, Ri (row stride LDR) get R[k][j] (upper) and R^{-1}[c][k]
-// (upper).  A bad pivot k zeroes row k of R and column k of R^{-1} (so column k
-// of Q), and drops row k from the later columns' elimination.  Returns true
-// if a pivot was bad.
-template <int LDS_, int LDR>
-__device__ __forceinline__ bool cholesky_wave(const double *S, const double *d0, double *R, double *Ri)
+// v += (lane K of each 16-lane row of l) b, for N values each of s and m
+// against the same l = s: one v_fmac_f64 with a DPP row broadcast per value.
+// (A DPP read needs two instructions after the write of its register: the
+// callers' order gives that inside a pivot, the trailing s_nop across pivots.)
+template <int K, int N>
+__device__ __forceinline__ void rank1_rows(double *s, double *m, double a, double b)
 {
-    constexpr int kW = 32;
-    const int lane = threadIdx.x & 63;
-    const bool aug = lane >= kW;
-    const int j = lane & (kW - 1);
-    double g[kW];
-#pragma unroll
-    for (int i = 0; i < kW; ++i) g[i] = aug ? (i == j ? 1.0 : 0.0) : S[i * LDS_ + j];
-    // The reference norms in registers before the elimination: read inside
-    // the loop, each would put an LDS latency on the serial chain (the loop's
-    // stores to R and Ri keep the compiler from hoisting them).
-    double dk[kW];
-#pragma unroll
-    for (int k = 0; k < kW; ++k) dk[k] = d0[k];
-    bool bad = false;
-#pragma unroll
-    for (int k = 0; k < kW; ++k) {
-        const double p = readlane_f64(g[k], k);
-        const double p0 = dk[k];
-        const bool ok = p0 > 0.0 && p > kPivotRel * p0 && p <= 1.7976931348623157e308;
-        bad |= !ok;
-        // 1/sqrt(p): hardware estimate and two Newton steps.
-        const double pp = ok ? p : 1.0;
-        double y = __builtin_amdgcn_rsq(pp);
-        y = y * fma(-0.5 * pp * y, y, 1.5);
-        y = y * fma(-0.5 * pp * y, y, 1.5);
-        const double inv = ok ? y : 0.0;
-        const double d = ok ? p * y : 0.0;
-        const double val = g[k] * inv;
-        if (aug)
-            Ri[j * LDR + k] = val;
-        else
-            R[k * LDR + j] = (j < k) ? 0.0 : (j == k ? d : val);
-        const double a = val * inv;  // row k of the trailing matrix (or of M) / p
-#pragma unroll
-        for (int i = k + 1; i < kW; ++i) g[i] = fma(-readlane_f64(g[i], k), a, g[i]);
+#define LATER_ROW(S, M)                                                                    \
+    "v_fmac_f64_dpp %" #M ", %" #S ", %[b] row_newbcast:%c[k] row_mask:0xf bank_mask:0xf\n\t" \
+    "v_fmac_f64_dpp %" #S ", %" #S ", %[a] row_newbcast:%c[k] row_mask:0xf bank_mask:0xf\n\t"
+    if constexpr (N == 1)
+        asm(LATER_ROW(0, 1) "s_nop 1" : "+v"(s[0]), "+v"(m[0]) : [a] "v"(a), [b] "v"(b), [k] "n"(K));
+    else if constexpr (N == 2)
+        asm(LATER_ROW(0, 2) LATER_ROW(1, 3) "s_nop 1"
+            : "+v"(s[0]), "+v"(s[1]), "+v"(m[0]), "+v"(m[1]) : [a] "v"(a), [b] "v"(b), [k] "n"(K));
+    else if constexpr (N == 3)
+        asm(LATER_ROW(0, 3) LATER_ROW(1, 4) LATER_ROW(2, 5) "s_nop 1"
+            : "+v"(s[0]), "+v"(s[1]), "+v"(s[2]), "+v"(m[0]), "+v"(m[1]), "+v"(m[2])
+            : [a] "v"(a), [b] "v"(b), [k] "n"(K));
+    else if constexpr (N == 4)
+        asm(LATER_ROW(0, 4) LATER_ROW(1, 5) LATER_ROW(2, 6) LATER_ROW(3, 7) "s_nop 1"
+            : "+v"(s[0]), "+v"(s[1]), "+v"(s[2]), "+v"(s[3]), "+v"(m[0]), "+v"(m[1]), "+v"(m[2]), "+v"(m[3])
+            : [a] "v"(a), [b] "v"(b), [k] "n"(K));
+    else if constexpr (N > 4) {
+        rank1_rows<K, 4>(s, m, a, b);
+        rank1_rows<K, N - 4>(s + 4, m + 4, a, b);
     }
-    return bad;
+#undef LATER_ROW
+}
+
+// Elimination of a 16 x 16 block S = L D L^T in LDS by one wave: U = D L^T,
+// M = L^{-1} and 1/sqrt(d_k), so that R = D^{-1/2} U and R^{-T} = D^{-1/2} M
+// (Gauss-Jordan on [S | I]).  Each 16-lane row of the wave holds all of it
+// (lane j: column j of the trailing matrix and of the identity's rows), so a
+// pivot's row is already in every lane and its multipliers are a DPP row
+// broadcast inside the multiply-add: no value crosses through scalar
+// registers.  Only 1/d_k is on the serial chain; the square roots are taken at
+// once afterwards, one per lane.
+// S: row stride LDS_; least[k]: what pivot k has to exceed.  U (row stride 16), M (row stride kLdM) get rows k, isq[k]
+// the scale; a bad pivot k gets scale 0 (which zeroes row k of R and column k
+// of R^{-1}, so column k of Q) and drops row k from the later columns'
+// elimination.  Returns true if a pivot was bad.
+constexpr int kLdM = 17;
+
+template <int K>
+__device__ __forceinline__ void eliminate16_from(double *s, double *m, const double *least)
+{
+    const double p = dpp_d<0x150 + K>(s[K]);  // row_newbcast:K
+    // 1/p: hardware estimate and two Newton steps.
+    double y = __builtin_amdgcn_rcp(p);
+    y = fma(fma(-p, y, 1.0), y, y);
+    y = fma(fma(-p, y, 1.0), y, y);
+    y = p > least[K] ? y : 0.0;
+    rank1_rows<K, 15 - K>(s + K + 1, m + K + 1, -(s[K] * y), -(m[K] * y));
+    if constexpr (K + 1 < 16) eliminate16_from<K + 1>(s, m, least);
+}
+
+template <int LDS_>
+__device__ __forceinline__ bool eliminate16_wave(const double *S, const double *least, double *U, double *M,
+                                                 double *isq)
+{
+    constexpr int kW = 16;
+    const int lane = threadIdx.x & 63, j = lane & (kW - 1);
+    double s[kW], m[kW], lk[kW];
+#pragma unroll
+    for (int i = 0; i < kW; ++i) {
+        s[i] = S[i * LDS_ + j];
+        m[i] = i == j ? 1.0 : 0.0;
+        lk[i] = least[i];
+    }
+    eliminate16_from<0>(s, m, lk);
+    if (lane < kW) {
+#pragma unroll
+        for (int i = 0; i < kW; ++i) {
+            U[i * kW + j] = s[i];
+            M[i * kLdM + j] = m[i];
+        }
+    }
+    // Lane j's own pivot; estimate of 1/sqrt and two Newton steps.
+    const double d = U[j * kW + j];
+    const bool ok = d > least[j] && d <= 1.7976931348623157e308;
+    const double p = ok ? d : 1.0;
+    double y = __builtin_amdgcn_rsq(p);
+    y = y * fma(-0.5 * p * y, y, 1.5);
+    y = y * fma(-0.5 * p * y, y, 1.5);
+    if (lane < kW) isq[j] = ok ? y : 0.0;
+    return __builtin_amdgcn_ballot_w64(!ok) != 0;
 }
 
 // G = R^T R and R^{-1} for the W x W Gram in LDS (Gs, row stride W + 1; R and
-// Ri row stride W).  W = 64 runs the blocked form with 32 x 32 blocks
-// G = [A B; B^T C]: A = R11^T R11, R12 = R11^{-T} B, C - R12^T R12 = R22^T R22,
-// R^{-1} = [R11^{-1}, -R11^{-1} R12 R22^{-1}; 0, R22^{-1}] (all FP64); a pivot
-// of the second block is compared with the diagonal of C.  Destroys Gs.
-// Called by every thread of the workgroup; returns (on thread 0) whether a
-// pivot was bad.
+// Ri row stride W), blocked by 16: the elimination of [G | I] with the
+// diagonal blocks on wave 0 (eliminate16_wave) and every other product on FP64
+// MFMA.  Step b: X_bb = R_bb^{-T}; R_bj = X_bb G_bj (j > b) and
+// X_bj = X_bb Y_bj (j < b); then G_ij -= R_bi^T R_bj (b < i <= j) and
+// Y_ij -= R_bi^T X_bj (i > b >= j).  X (= R^{-T}) and Y share the lower
+// blocks of Gs; Ris holds U, M and the scales of the current step until the
+// end.  Wave 0 updates the next diagonal block and goes on to its
+// elimination while the other waves update the rest, so the serial path is
+// the W / 16 eliminations and one product before and after each.  A pivot is
+// compared with the diagonal of G.  Destroys Gs.  Called by every thread of
+// the workgroup; returns (on wave 0) whether a pivot was bad.
+// Bound: the dependent FP64 chain of the pivots (about 100 cycles each) and
+// the issue of the rank-1 rows beside it.  W = 64: 10 us, where two 32 x 32
+// one-wave eliminations, fully unrolled with scalar broadcasts and each
+// pivot's square root on the chain, took 19 us (a first-pass leaf of 8192 x 64:
+// factor and apply 30 -> 21 us).
 template <int W> __device__ __forceinline__ bool factor(double *Gs, double *Rs, double *Ris, double *d0)
 {
-    constexpr int LDG = Shape<W>::LDG;
-    const int t = threadIdx.x;
-    if (t < W) d0[t] = Gs[t * LDG + t];
+    constexpr int LDG = Shape<W>::LDG, NB = W / 16;
+    const int t = threadIdx.x, lane = t & 63, wv = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int li = lane & 15, lk = lane >> 4;
+    double *U = Ris, *M = Ris + 256, *isq = Ris + 256 + 16 * kLdM;
+    static_assert(256 + 16 * kLdM + 16 <= W * W, "scratch in Ris");
+    if (t < W) {
+        const double g = Gs[t * LDG + t];
+        d0[t] = g > 0.0 ? kPivotRel * g : __longlong_as_double(0x7ff0000000000000ll);
+    }
+    // Zero blocks of R below the diagonal ones.
+    for (int e = t; e < W * W; e += kThreads)
+        if (e / W / 16 > e % W / 16) Rs[e] = 0.0;
     __syncthreads();
+    // One 16 x 16 tile: T = c + a b over k = 0 .. 15 (v_mfma_f64_16x16x4f64: lane
+    // l, entry r of the result is tile element (l / 16 + 4 r, l % 16)).
+    // a(x, k) by the caller; b[k][y] at B + k ldb + y.
+    auto product = [&](const double (&av)[4], const double *B, int ldb, doublex4 c) {
+        double bv[4];
+#pragma unroll
+        for (int s = 0; s < 4; ++s) bv[s] = B[(4 * s + lk) * ldb + li];
+#pragma unroll
+        for (int s = 0; s < 4; ++s) c = __builtin_amdgcn_mfma_f64_16x16x4f64(av[s], bv[s], c, 0, 0, 0);
+        return c;
+    };
+    // Tile (i, j) of the trailing update of step b: both halves read row b of
+    // R (R_bj) or of X (X_bj, whose blocks lie in Gs).
+    auto trailing = [&](int b, int i, int j) {
+        double *T = Gs + 16 * i * LDG + 16 * j;
+        doublex4 c = doublex4{0.0, 0.0, 0.0, 0.0};
+        if (!(i > j && j == b)) {  // Y_ib starts here
+#pragma unroll
+            for (int r = 0; r < 4; ++r) c[r] = T[(lk + 4 * r) * LDG + li];
+        }
+        double av[4];
+#pragma unroll
+        for (int s = 0; s < 4; ++s) av[s] = -Rs[(16 * b + 4 * s + lk) * W + 16 * i + li];
+        c = i <= j ? product(av, Rs + 16 * b * W + 16 * j, W, c) : product(av, Gs + 16 * b * LDG + 16 * j, LDG, c);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) T[(lk + 4 * r) * LDG + li] = c[r];
+    };
     bool bad = false;
-    if (t < 64) bad = cholesky_wave<LDG, W>(Gs, d0, Rs, Ris);
-    if constexpr (W == 64) {
+#pragma unroll 1
+    for (int b = 0; b < NB; ++b) {
+        if (wv == 0) {
+            if (b > 0) trailing(b - 1, b, b);
+            bad |= eliminate16_wave<LDG>(Gs + 16 * b * LDG + 16 * b, d0 + 16 * b, U, M, isq);
+        } else if (b > 0) {
+            int n = 0;
+#pragma unroll 1
+            for (int i = b; i < NB; ++i)
+#pragma unroll 1
+                for (int j = 0; j < NB; ++j)
+                    if ((i <= j || j < b) && !(i == b && j == b)) {
+                        if (n == wv - 1) trailing(b - 1, i, j);
+                        n = n == 2 ? 0 : n + 1;
+                    }
+        }
         __syncthreads();
-        // The four 32 x 32 x 32 products below run on FP64 MFMA: wave w makes
-        // the 16 x 16 tile (w / 2, w % 2) of each, over the full k range (the
-        // triangular factors' zero halves are stored, so the sums are the
-        // same).  Result layout (v_mfma_f64_16x16x4f64): lane l, entry r holds
-        // tile element (l / 16 + 4 r, l % 16).
-        const int lane = t & 63, wv = t >> 6, ti = 16 * (wv >> 1), tj = 16 * (wv & 1);
-        const int li = lane & 15, lk = lane >> 4;
-        auto product = [&](auto a, auto b, doublex4 c) {
-#pragma unroll
-            for (int s = 0; s < 8; ++s)
-                c = __builtin_amdgcn_mfma_f64_16x16x4f64(a(ti + li, 4 * s + lk), b(4 * s + lk, tj + li), c, 0, 0, 0);
-            return c;
-        };
-        const doublex4 zero = doublex4{0.0, 0.0, 0.0, 0.0};
-        // R12 = R11^{-T} B -> Rs[i][32 + j]; zero lower-left blocks.
-        {
-            const doublex4 c = product([&](int i, int k) { return Ris[k * W + i]; },
-                                       [&](int k, int j) { return Gs[k * LDG + 32 + j]; }, zero);
-#pragma unroll
-            for (int r = 0; r < 4; ++r) Rs[(ti + lk + 4 * r) * W + 32 + tj + li] = c[r];
-            const int j = t & 31, i0 = t >> 5;
+        if (wv == 3) {
+            // R_bb and X_bb (over G_bb).
 #pragma unroll
             for (int u = 0; u < 4; ++u) {
-                const int i = i0 + 8 * u;
-                Rs[(32 + i) * W + j] = 0.0;
-                Ris[(32 + i) * W + j] = 0.0;
+                const int k = lk + 4 * u;
+                const double s = isq[k];
+                Rs[(16 * b + k) * W + 16 * b + li] = li < k ? 0.0 : U[k * 16 + li] * s;
+                Gs[(16 * b + k) * LDG + 16 * b + li] = M[k * kLdM + li] * s;
             }
+        } else if (wv < NB - 1) {
+            // Row b of R and of X: block j on wave (j - b - 1) mod NB, so that
+            // the next diagonal block's factor R_b,b+1 is wave 0's.
+            const int j = (b + 1 + wv) % NB;
+            double av[4];
+#pragma unroll
+            for (int s = 0; s < 4; ++s) av[s] = M[li * kLdM + 4 * s + lk] * isq[li];
+            const doublex4 c = product(av, Gs + 16 * b * LDG + 16 * j, LDG, doublex4{0.0, 0.0, 0.0, 0.0});
+            double *T = j > b ? Rs + 16 * b * W + 16 * j : Gs + 16 * b * LDG + 16 * j;
+            const int ld = j > b ? W : LDG;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) T[(lk + 4 * r) * ld + li] = c[r];
         }
         __syncthreads();
-        // S = C - R12^T R12, in place over C.
-        {
-            doublex4 c;
-#pragma unroll
-            for (int r = 0; r < 4; ++r) c[r] = Gs[(32 + ti + lk + 4 * r) * LDG + 32 + tj + li];
-            c = product([&](int i, int k) { return -Rs[k * W + 32 + i]; },
-                        [&](int k, int j) { return Rs[k * W + 32 + j]; }, c);
-            __syncthreads();  // every wave has read C before any writes S over it
-#pragma unroll
-            for (int r = 0; r < 4; ++r) Gs[(32 + ti + lk + 4 * r) * LDG + 32 + tj + li] = c[r];
-        }
-        __syncthreads();
-        if (t < 64) bad |= cholesky_wave<LDG, W>(Gs + 32 * LDG + 32, d0 + 32, Rs + 32 * W + 32, Ris + 32 * W + 32);
-        __syncthreads();
-        // T = R12 R22^{-1} -> over A (Gs[i][j]).
-        {
-            const doublex4 c = product([&](int i, int k) { return Rs[i * W + 32 + k]; },
-                                       [&](int k, int j) { return Ris[(32 + k) * W + 32 + j]; }, zero);
-#pragma unroll
-            for (int r = 0; r < 4; ++r) Gs[(ti + lk + 4 * r) * LDG + tj + li] = c[r];
-        }
-        __syncthreads();
-        // R^{-1}[i][32 + j] = -(R11^{-1} T)[i][j].  A bad pivot k leaves, as
-        // in one block, row k of R and column k of R^{-1} zero.
-        {
-            const doublex4 c = product([&](int i, int k) { return -Ris[i * W + k]; },
-                                       [&](int k, int j) { return Gs[k * LDG + j]; }, zero);
-#pragma unroll
-            for (int r = 0; r < 4; ++r) Ris[(ti + lk + 4 * r) * W + 32 + tj + li] = c[r];
-        }
+    }
+    // R^{-1} = X^T, zeros below the diagonal.
+    for (int e = t; e < W * W; e += kThreads) {
+        const int i = e / W, j = e % W;
+        Ris[e] = i <= j ? Gs[j * LDG + i] : 0.0;
     }
     return bad;
 }

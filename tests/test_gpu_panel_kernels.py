@@ -48,3 +48,26 @@ def test_tsqr_apply_levels(later, oracle, m, w, fp64):
     Qo, Ro = oracle.caqr32(A)
     assert oracle.rel_err(R, Ro) < 2e-6 and oracle.rel_err(Q, Qo) < 4e-6
     assert oracle.orth(Q) < (2e-6 if fp64 else 4e-6) * np.sqrt(w)
+
+
+# The 16-blocked Cholesky factor: dependent columns (a zero column, a repeated
+# one) at the edges of its blocks, widths that end inside each block, on the
+# fused launch and (200000 rows) the separate factor launch.  The dependent
+# column of Q is zero, the rest orthonormal, A = QR still holds: the bounds of
+# the other wide-leaf tests.
+@pytest.mark.parametrize("m", [1500, 200000])
+@pytest.mark.parametrize("w,dup", [(17, (None, 16)), (16, (0, 15)), (48, (31, 32)), (64, (None, 0)), (64, (15, 16)),
+                                   (64, (5, 63)), (33, (None, 32)), (49, (47, 48)), (32, (2, 17))])
+def test_cholesky_leaf_blocks_breakdown(later, oracle, m, w, dup):
+    A = oracle.gen_uniform(m, w, 7, 3)
+    A[:, dup[1]] = 0.0 if dup[0] is None else A[:, dup[0]]
+    X = _dev(later, A)
+    o = later.opts("mixed")
+    work = later.workspace(m, w, o)
+    R = later.rgsqrf(X, o=o, work=work)
+    torch.cuda.synchronize()
+    assert later.read_status(work) & 1
+    Q, R = _np(X), _np(R)
+    keep = [j for j in range(w) if j != dup[1]]
+    assert np.all(Q[:, dup[1]] == 0) and np.isfinite(Q).all() and np.isfinite(R).all()
+    assert oracle.orth(Q[:, keep]) < 2e-6 * np.sqrt(w) and oracle.backward(A, Q, R) < 1e-6
