@@ -141,3 +141,12 @@ int gemm_nn(hipStream_t s, int prec, int M, int N, int K, float alpha, const flo
 
 // e[j] such that max |X(:,j)| 2^e[j] lies in [2^14, 2^15).
 int gemm_colexp(hipStream_t s, int m, int n, const float *X, int64_t ldx, int *e, int *launches);
+
+// FP32 products of narrow nodes (gemm_narrow.hip), the bits of the general
+// kernel; false: the shape is not theirs and nothing was launched.  The
+// projection writes split p's partial at partial + p n1 n2 (nullptr: C, one
+// split); the update is B += alpha Q C (f64: the sum in FP64).
+bool gemm_proj_narrow(hipStream_t s, int m, int n1, int n2, const float *Q, int64_t ldq, const float *B, int64_t ldb,
+                      float *C, int64_t ldc, int nsplit, int kper, float *partial);
+bool gemm_update_narrow(hipStream_t s, int M, int N, int K, float alpha, const float *Q, int64_t ldq, const float *C,
+                        int64_t ldc, float *B, int64_t ldb, bool f64);

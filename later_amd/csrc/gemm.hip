@@ -1129,8 +1129,9 @@ __global__ __launch_bounds__(NT) void gemm_grouped_kernel(const GemmArgs *args, 
     gemm_body<PREC, BM, BN, AKM, CH64, false>(g, t.y, t.z, t.w);
 }
 
-// C = sum over splits (fixed order, FP64) of the partials; 16 loads in
-// flight per thread (the sum itself stays sequential in p).
+// C = sum over splits (fixed order, FP64) of the partials; 16 or 32 loads in
+// flight per thread (the sum itself stays sequential in p): a round of loads
+// costs a memory latency, so up to 32 splits take one.
 template <bool F64>
 __global__ void splitk_reduce_kernel(int M, int N, int nsplit, const void *partial, float *C, int64_t ldc)
 {
@@ -1138,19 +1139,23 @@ __global__ void splitk_reduce_kernel(int M, int N, int nsplit, const void *parti
     const int64_t tot = (int64_t)M * N;
     if (idx >= tot) return;
     const int row = (int)(idx % M), col = (int)(idx / M);
-    constexpr int kB = 16;
     double s = 0.0;
-    for (int p0 = 0; p0 < nsplit; p0 += kB) {
-        double v[kB];
+    auto add = [&](auto batch) {
+        constexpr int kB = decltype(batch)::value;
+        for (int p0 = 0; p0 < nsplit; p0 += kB) {
+            double v[kB];
 #pragma unroll
-        for (int u = 0; u < kB; ++u) {
-            const int64_t off = (int64_t)min(p0 + u, nsplit - 1) * tot + idx;
-            v[u] = F64 ? ((const double *)partial)[off] : (double)((const float *)partial)[off];
+            for (int u = 0; u < kB; ++u) {
+                const int64_t off = (int64_t)min(p0 + u, nsplit - 1) * tot + idx;
+                v[u] = F64 ? ((const double *)partial)[off] : (double)((const float *)partial)[off];
+            }
+#pragma unroll
+            for (int u = 0; u < kB; ++u)
+                if (p0 + u < nsplit) s += v[u];
         }
-#pragma unroll
-        for (int u = 0; u < kB; ++u)
-            if (p0 + u < nsplit) s += v[u];
-    }
+    };
+    if (nsplit <= 16) add(std::integral_constant<int, 16>());
+    else add(std::integral_constant<int, 32>());
     C[(int64_t)col * ldc + row] = (float)s;
 }
 
@@ -1661,7 +1666,12 @@ int gemm_proj(hipStream_t s, int prec, int m, int n1, int n2, const float *Q, in
         g.b_exp = (const int *)((const char *)bh->p + bh->ls);
     }
     const int tok = prof_start(s);
-    int rc = ch64 ? dispatch<true, true>(s, prec, g, ns, small) : dispatch<true, false>(s, prec, g, ns, small);
+    int rc = LATER_OK;
+    if (prec == GEMM_F32 && !ch64 && !b_exp && a_exp == 0 &&
+        gemm_proj_narrow(s, m, n1, n2, Q, ldq, B, ldb, C, ldc, ns, kp, (float *)g.partial))
+        rc = hipGetLastError() == hipSuccess ? LATER_OK : LATER_ERR_DEVICE;
+    else
+        rc = ch64 ? dispatch<true, true>(s, prec, g, ns, small) : dispatch<true, false>(s, prec, g, ns, small);
     // Unfolded hi/lo projections on pre-split pieces run the updates' 256-row
     // streaming kernel: they are timed in its class.
     const bool x3 = prec == GEMM_F16X3 && !ch64 && !small && g.Ah && g.Bh;
@@ -1706,7 +1716,12 @@ int gemm_nn(hipStream_t s, int prec, int M, int N, int K, float alpha, const flo
     // 256 CUs, run the smaller tiles.
     const bool small = (N <= 64) || ceil_div64(M, 128) * ceil_div64(N, 128) < 256;
     const int tok = prof_start(s);
-    int rc = dispatch<false, false>(s, prec, g, 1, small);
+    int rc = LATER_OK;
+    if (prec == GEMM_F32 && !tri && !b_exp && a_exp == 0 &&
+        gemm_update_narrow(s, M, N, K, alpha, A, lda, B, ldb, C, ldc, f64))
+        rc = hipGetLastError() == hipSuccess ? LATER_OK : LATER_ERR_DEVICE;
+    else
+        rc = dispatch<false, false>(s, prec, g, 1, small);
     const bool x3 = prec == GEMM_F16X3 && !small && g.Ah && g.Bh;
     prof_stop(tok, s, x3 ? PROF_UPDATE_X3 : PROF_GEMM_UPDATE, tri ? (double)M * N * K / 3.0 : 2.0 * M * N * K,
               4.0 * ((double)M * K + 2.0 * M * N + (double)K * N));

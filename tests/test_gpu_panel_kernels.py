@@ -71,3 +71,20 @@ def test_cholesky_leaf_blocks_breakdown(later, oracle, m, w, dup):
     keep = [j for j in range(w) if j != dup[1]]
     assert np.all(Q[:, dup[1]] == 0) and np.isfinite(Q).all() and np.isfinite(R).all()
     assert oracle.orth(Q[:, keep]) < 2e-6 * np.sqrt(w) and oracle.backward(A, Q, R) < 1e-6
+
+
+# FP32 products of narrow nodes: tile edges, K blocks of 128 and splits, any
+# leading dimension (dword-aligned vector loads).  Each product is a chain of K
+# fused multiply-adds (and a sum of split partials in FP64), so an element is
+# within (K + 2) 2^-24 of its terms' magnitudes.
+@pytest.mark.parametrize("m", [1, 15, 17, 128, 129, 257, 4099])
+@pytest.mark.parametrize("n1,n2,pad", [(1, 1, 0), (31, 33, 1), (32, 32, 2), (64, 96, 3), (128, 127, 0), (65, 128, 1)])
+def test_narrow_products(later, oracle, m, n1, n2, pad):
+    u = 2.0 ** -24
+    Q, B, C = oracle.gen_uniform(m, n1, 1, 1), oracle.gen_uniform(m, n2, 2, 2), oracle.gen_uniform(n1, n2, 3, 3)
+    q, b, c = _dev(later, Q, pad), _dev(later, B, pad), _dev(later, C, pad)
+    P = _np(later.gemm_proj(q, b, later.colmajor(n1, n2, ld=n1 + pad), later.GEMM_F32))
+    Q, B, C = Q.astype(np.float64), B.astype(np.float64), C.astype(np.float64)
+    assert np.all(np.abs(P - Q.T @ B) <= (m + 2) * u * (np.abs(Q).T @ np.abs(B)) + 1e-45)
+    U = _np(later.gemm_update(q, c, b, later.GEMM_F32))
+    assert np.all(np.abs(U - (B - Q @ C)) <= (n1 + 2) * u * (np.abs(Q) @ np.abs(C) + np.abs(B)) + 1e-45)
