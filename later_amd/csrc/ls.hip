@@ -3,61 +3,104 @@
 // Q^T B is the node projection GEMM (gemm.hip).  The triangular solve is a
 // blocked back substitution standing in for the reference's recursive TRSM
 // (BLAS/later_rtrsm.cu:75-187): one workgroup per right-hand side keeps the
-// column in LDS in FP64; each 64-row diagonal block is solved by one wave with
-// the block held in registers (lane i owns row i, x_r is broadcast by a
-// shuffle), then the rows above are updated by all waves with FP64 sums.
+// column in LDS in FP64 and works up R in 64-row blocks.
 #include "common.h"
 #include "gemm.h"
 
 namespace {
 
 constexpr int TB = 64;          // diagonal block
-constexpr int NT = 256;
+constexpr int kWaves = 8;
+constexpr int NT = 64 * kWaves;
 constexpr int kMaxN = 8192;     // FP64 column in LDS: 64 KiB
 
+// Block b's rows need the products with every later block's x.  While wave 0
+// solves block b (lane i owns row i of the diagonal block in registers, x_r is
+// read from lane r after one multiplication by the reciprocal of its
+// diagonal), the other waves sum block b - 1's products with the blocks after
+// b, and every wave's share of block b's own columns is already in flight; one
+// barrier after x_b is known those are added, and wave 0 goes on.
+// Bound: wave 0's chain, 64 x (multiply, broadcast, multiply-add) a block: 512
+// unknowns 49 us, where loads and a division on the chain took 398.
+template <int NMAX>
 __global__ __launch_bounds__(NT) void trsm_upper_kernel(int n, const float *R, int64_t ldr, float *B, int64_t ldb,
                                                         int *status)
 {
-    extern __shared__ double x[];
+    __shared__ double x[NMAX], part[kWaves][TB];
     float *b = B + (int64_t)blockIdx.x * ldb;
-    for (int i = threadIdx.x; i < n; i += NT) x[i] = (double)b[i];
-    __syncthreads();
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int nblk = (n + TB - 1) / TB;
+    // Wave 0: row `lane` of the diagonal block (its part right of the
+    // diagonal) and the diagonal entry.
+    float dn[TB], diag_n = 1.0f;
+    auto load_diag = [&](int j0) {
+        const int row = min(j0 + lane, n - 1);
+#pragma unroll
+        for (int r = 0; r < TB; ++r) dn[r] = R[row + (int64_t)min(j0 + r, n - 1) * ldr];
+        diag_n = R[row + (int64_t)row * ldr];
+    };
+    if (wave == 0) load_diag((nblk - 1) * TB);
+    for (int i = threadIdx.x; i < n; i += NT) x[i] = (double)b[i];
+    part[wave][lane] = 0.0;
+    __syncthreads();
+    constexpr int kShare = TB / kWaves;
     for (int blk = nblk - 1; blk >= 0; --blk) {
-        const int j0 = blk * TB;
-        const int jn = min(TB, n - j0);
-        if (wave == 0) {
-            // Rows j0 .. j0+jn-1: lane i owns row j0+i.
-            double xi = (lane < jn) ? x[j0 + lane] : 0.0;
-            for (int r = jn - 1; r >= 0; --r) {
-                const float drr = R[(j0 + r) + (int64_t)(j0 + r) * ldr];
-                double xr = __shfl(xi, r, 64);
-                if (!(drr != 0.0f) && lane == 0 && status) atomicOr(status, 2);
-                xr = (drr != 0.0f) ? xr / (double)drr : 0.0;
-                if (lane == r) xi = xr;
-                if (lane < r) xi -= (double)R[(j0 + lane) + (int64_t)(j0 + r) * ldr] * xr;
+        const int j0 = blk * TB, jn = min(TB, n - j0);
+        const int up = j0 - TB + lane;  // this lane's row of the block above
+        float f[kShare];
+        double acc = 0.0;
+        if (blk > 0) {
+#pragma unroll
+            for (int q = 0; q < kShare; ++q) {
+                const int c = kShare * wave + q;
+                const float v = R[up + (int64_t)(j0 + min(c, jn - 1)) * ldr];
+                f[q] = c < jn ? v : 0.0f;
             }
-            if (lane < jn) x[j0 + lane] = xi;
+        }
+        if (wave == 0) {
+            float d[TB];
+#pragma unroll
+            for (int r = 0; r < TB; ++r) d[r] = lane < r ? dn[r] : 0.0f;
+            const float diag = diag_n;
+            if (blk > 0) load_diag(j0 - TB);
+            double xi = lane < jn ? x[j0 + lane] : 0.0;
+#pragma unroll
+            for (int w = 0; w < kWaves; ++w) xi -= part[w][lane];
+            if (!(diag != 0.0f) && lane < jn && status) atomicOr(status, 2);
+            const double inv = diag != 0.0f ? 1.0 / (double)diag : 0.0;
+            double res = 0.0;
+#pragma unroll
+            for (int r = TB - 1; r >= 0; --r) {
+                if (r < jn) {
+                    const double xr = readlane_d(xi * inv, r);
+                    res = lane == r ? xr : res;
+                    xi = fma(-(double)d[r], xr, xi);
+                }
+            }
+            if (lane < jn) x[j0 + lane] = res;
+        } else if (blk > 0) {
+            constexpr int kU = 8;
+            for (int c0 = j0 + jn + wave - 1; c0 < n; c0 += kU * (kWaves - 1)) {
+                float v[kU];
+#pragma unroll
+                for (int u = 0; u < kU; ++u) v[u] = R[up + (int64_t)min(c0 + u * (kWaves - 1), n - 1) * ldr];
+#pragma unroll
+                for (int u = 0; u < kU; ++u) {
+                    const int c = c0 + u * (kWaves - 1);
+                    if (c < n) acc = fma((double)v[u], x[c], acc);
+                }
+            }
         }
         __syncthreads();
-        // x[0:j0] -= R[0:j0, j0:j0+jn] x[j0:j0+jn]
-        for (int i = threadIdx.x; i < j0; i += NT) {
-            double s = 0.0;
-            for (int c = 0; c < jn; ++c) s += (double)R[i + (int64_t)(j0 + c) * ldr] * x[j0 + c];
-            x[i] -= s;
+        if (blk > 0) {
+#pragma unroll
+            for (int q = 0; q < kShare; ++q)
+                if (kShare * wave + q < jn) acc = fma((double)f[q], x[j0 + kShare * wave + q], acc);
+            part[wave][lane] = acc;
         }
         __syncthreads();
     }
     for (int i = threadIdx.x; i < n; i += NT) b[i] = (float)x[i];
-}
-
-__global__ void copy_kernel(int m, int n, const float *X, int64_t ldx, float *Y, int64_t ldy)
-{
-    const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= (int64_t)m * n) return;
-    const int i = (int)(idx % m), j = (int)(idx / m);
-    Y[i + (int64_t)j * ldy] = X[i + (int64_t)j * ldx];
 }
 
 } // namespace
@@ -65,7 +108,12 @@ __global__ void copy_kernel(int m, int n, const float *X, int64_t ldx, float *Y,
 int trsm_upper(hipStream_t s, int n, int k, const float *R, int64_t ldr, float *B, int64_t ldb, int *status)
 {
     if (n < 1 || k < 1 || n > kMaxN) return LATER_ERR_SHAPE;
-    hipLaunchKernelGGL(trsm_upper_kernel, dim3(k), dim3(NT), sizeof(double) * n, s, n, R, ldr, B, ldb, status);
+    // The smaller column array leaves room for several workgroups a CU (servers
+    // solve on several streams at once).
+    if (n <= 1024)
+        hipLaunchKernelGGL(trsm_upper_kernel<1024>, dim3(k), dim3(NT), 0, s, n, R, ldr, B, ldb, status);
+    else
+        hipLaunchKernelGGL(trsm_upper_kernel<kMaxN>, dim3(k), dim3(NT), 0, s, n, R, ldr, B, ldb, status);
     HIP_OK(hipGetLastError());
     return LATER_OK;
 }

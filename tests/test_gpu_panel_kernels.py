@@ -88,3 +88,27 @@ def test_narrow_products(later, oracle, m, n1, n2, pad):
     assert np.all(np.abs(P - Q.T @ B) <= (m + 2) * u * (np.abs(Q).T @ np.abs(B)) + 1e-45)
     U = _np(later.gemm_update(q, c, b, later.GEMM_F32))
     assert np.all(np.abs(U - (B - Q @ C)) <= (n1 + 2) * u * (np.abs(Q) @ np.abs(C) + np.abs(B)) + 1e-45)
+
+
+# Triangular solve at the edges of its 64-row blocks and of its two column
+# arrays, and with a zero on the diagonal (its unknown is 0).  The sums are FP64
+# and x is rounded to FP32 once, so the residual is within 2^-24 (plus n FP64
+# roundings) of |R| |x| in every component.
+@pytest.mark.parametrize("n,k", [(1, 1), (63, 2), (65, 1), (129, 3), (1024, 3), (1025, 1)])
+@pytest.mark.parametrize("zero", [False, True])
+def test_trsm_upper_blocks(later, oracle, n, k, zero):
+    R = np.triu(oracle.gen_uniform(n, n, 4, 4)) + 4.0 * np.sqrt(n) * np.eye(n, dtype=np.float32)
+    R = R.astype(np.float32)
+    B = oracle.gen_uniform(n, k, 5, 5)
+    j = n // 2
+    if zero:
+        R[j, j] = 0.0
+    X = _dev(later, B, 1)
+    later.trsm_upper(_dev(later, R, 1), X)
+    X = _np(X).astype(np.float64)
+    rows = [i for i in range(n) if not (zero and i == j)]
+    if zero:
+        assert np.all(X[j] == 0.0)
+    R = R.astype(np.float64)
+    res = np.abs(R @ X - B)[rows]
+    assert np.all(res <= (2.0 ** -24 + n * 2.0 ** -50) * (np.abs(R) @ np.abs(X))[rows] + 1e-30)
