@@ -33,25 +33,35 @@ constexpr int kMaxRows = 320;             // rows of a block: 256, or up to 256 
 __device__ __forceinline__ bool norm_of(float s, float &nrm, float &inv)
 {
     const unsigned u = __builtin_amdgcn_readfirstlane(__float_as_uint(s));
-    if (u - 0x10000000u < 0x6E000000u - 0x10000000u) {  // 2^-95 <= s < 2^93
-        const float y = __builtin_amdgcn_sqrtf(s);
-        float r = __builtin_amdgcn_rsqf(s);
-        const float yd = __uint_as_float(__float_as_uint(y) - 1u), yu = __uint_as_float(__float_as_uint(y) + 1u);
-        const float ed = fmaf(-yd, y, s), eu = fmaf(-yu, y, s);
-        nrm = ed <= 0.0f ? yd : y;
-        nrm = eu > 0.0f ? yu : nrm;
+    const float y = __builtin_amdgcn_sqrtf(s);
+    float r = __builtin_amdgcn_rsqf(s);
+    const float yd = __uint_as_float(__float_as_uint(y) - 1u), yu = __uint_as_float(__float_as_uint(y) + 1u);
+    const float ed = fmaf(-yd, y, s), eu = fmaf(-yu, y, s);
+    nrm = ed <= 0.0f ? yd : y;
+    nrm = eu > 0.0f ? yu : nrm;
 #pragma unroll
-        for (int i = 0; i < 3; ++i) r = fmaf(fmaf(-nrm, r, 1.0f), r, r);
-        inv = r;
-        return true;
-    }
+    for (int i = 0; i < 3; ++i) r = fmaf(fmaf(-nrm, r, 1.0f), r, r);
+    inv = r;
+    if (__builtin_expect(u - 0x10000000u < 0x6E000000u - 0x10000000u, 1)) return true;  // 2^-95 <= s < 2^93
     nrm = sqrtf(s);
     const bool ok = (nrm > 0.0f) && (nrm < INFINITY);
     inv = ok ? 1.0f / nrm : 0.0f;
     return ok;
 }
+// FP64: the reciprocal root by two Newton steps from the estimate and the root
+// from it with one correction, each within an ulp or two of FP64 (Q and R are
+// rounded to FP32 once afterwards).
 __device__ __forceinline__ bool norm_of(double s, double &nrm, double &inv)
 {
+    const unsigned e = (unsigned)__builtin_amdgcn_readfirstlane(__double2hiint(s)) >> 20;
+    double y = __builtin_amdgcn_rsq(s);
+    const double h = 0.5 * s;
+    y = y * fma(-h * y, y, 1.5);
+    y = y * fma(-h * y, y, 1.5);
+    const double g = s * y;
+    nrm = fma(fma(-g, g, s), 0.5 * y, g);
+    inv = y;
+    if (__builtin_expect(e - 23u < 2000u, 1)) return true;  // positive, 2^-1000 <= s < 2^1000
     nrm = sqrt(s);
     const bool ok = (nrm > 0.0) && (nrm < INFINITY);
     inv = ok ? 1.0 / nrm : 0.0;
@@ -68,8 +78,8 @@ __device__ __forceinline__ bool norm_of(double s, double &nrm, double &inv)
 // their order are those of plain MGS: for k = 0, 1, ...: d = q_k . a,
 // a -= q_k d.
 // Bound: the serial chain of w norms (dot, wave sum, square root, reciprocal):
-// 13 us for 256 x 32, where one barrier per column and a column dealt to
-// every eighth wave took 24 us (same bits; FP64 sums 22 and 30 us).
+// 12 us for 256 x 32, where one barrier per column and a column dealt to
+// every eighth wave took 24 us (same bits; FP64 sums 21 and 30 us).
 // RPL: rows per lane, 4 for blocks of up to 256 rows, 5 with a merged tail.
 template <typename Acc, int RPL>
 __device__ __forceinline__ void mgs_block_body(int m, int w, float *A, int64_t lda, float *Rout, int64_t ldr,
@@ -105,76 +115,120 @@ __device__ __forceinline__ void mgs_block_body(int m, int w, float *A, int64_t l
     __syncthreads();
 
     // Columns C0 .. of this wave: d = q . a, a -= q d.
-    auto project = [&](const float (&q)[RPL], auto first, Acc *dout) {
-        constexpr int C0 = decltype(first)::value, N = kCPW - C0;
-        Acc d[N];
+    auto dot = [&](const float (&q)[RPL], int c) -> Acc {
+        Acc d = (Acc)q[0] * (Acc)a[c][0];
 #pragma unroll
-        for (int c = 0; c < N; ++c) d[c] = (Acc)q[0] * (Acc)a[C0 + c][0];
+        for (int t = 1; t < RPL; ++t) d = fma((Acc)q[t], (Acc)a[c][t], d);
+        return d;
+    };
+    auto subtract = [&](const float (&q)[RPL], int c, Acc d) {
 #pragma unroll
-        for (int t = 1; t < RPL; ++t)
-#pragma unroll
-            for (int c = 0; c < N; ++c) d[c] = fma((Acc)q[t], (Acc)a[C0 + c][t], d[c]);
-        wave_sums(d);
-#pragma unroll
-        for (int c = 0; c < N; ++c) {
-#pragma unroll
-            for (int t = 0; t < RPL; ++t) {
-                a[C0 + c][t] = (float)fma(-(Acc)q[t], d[c], (Acc)a[C0 + c][t]);
-                asm volatile("" : "+v"(a[C0 + c][t]));  // here, not sunk below the stores that follow
-            }
-            dout[C0 + c] = d[c];
+        for (int t = 0; t < RPL; ++t) {
+            a[c][t] = (float)fma(-(Acc)q[t], d, (Acc)a[c][t]);
+            asm volatile("" : "+v"(a[c][t]));  // here, not sunk below the stores that follow
         }
+    };
+    auto norm_terms = [&](int c) -> Acc {
+        Acc s = (Acc)a[c][1] * (Acc)a[c][1];
+        s = fma((Acc)a[c][0], (Acc)a[c][0], s);
+#pragma unroll
+        for (int t = 2; t < RPL; ++t) s = fma((Acc)a[c][t], (Acc)a[c][t], s);
+        return s;
+    };
+    // All of them by q.
+    auto project = [&](const float (&q)[RPL], Acc *d) {
+        Acc v[kCPW];
+#pragma unroll
+        for (int c = 0; c < kCPW; ++c) v[c] = dot(q, c);
+        wave_sums(v);
+#pragma unroll
+        for (int c = 0; c < kCPW; ++c) {
+            subtract(q, c, v[c]);
+            d[c] = v[c];
+        }
+    };
+    // Columns C0 .. by q, the next pivot's column C0 first: its squared norm is
+    // summed together with the other columns' products.  Returns that norm.
+    auto project_next = [&](const float (&q)[RPL], auto first, Acc *d) -> Acc {
+        constexpr int C0 = decltype(first)::value, N = kCPW - C0;
+        Acc h[1] = {dot(q, C0)};
+        wave_sums(h);
+        subtract(q, C0, h[0]);
+        d[C0] = h[0];
+        Acc v[N];
+        v[0] = norm_terms(C0);
+#pragma unroll
+        for (int c = 1; c < N; ++c) v[c] = dot(q, C0 + c);
+        wave_sums(v);
+#pragma unroll
+        for (int c = 1; c < N; ++c) {
+            subtract(q, C0 + c, v[c]);
+            d[C0 + c] = v[c];
+        }
+        return v[0];
     };
     auto load_q = [&](float (&q)[RPL], int k) {
 #pragma unroll
         for (int t = 0; t < RPL; ++t) q[t] = qs[k][lane + 64 * t];
     };
+    auto count = [&]() { return __hip_atomic_load(&published, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP); };
+    // The count and, behind it in the same LDS queue, q_k: valid when the count
+    // says so.
+    auto peek = [&](float (&q)[RPL], int k) -> int {
+        const int n = count();
+        asm volatile("" ::: "memory");
+        load_q(q, k);
+        asm volatile("" ::: "memory");
+        return n;
+    };
+    // q_k, waiting for it: the wave whose turn is next reads it with every
+    // look at the count, the ones behind it only look.
+    auto take = [&](float (&q)[RPL], int k) {
+        if (c0 - k > kCPW)
+            while (__builtin_amdgcn_readfirstlane(count()) <= k) {}
+        asm volatile("" ::: "memory");
+        while (__builtin_amdgcn_readfirstlane(peek(q, k)) <= k) {}
+    };
 
+    Acc s0 = 0;
     if (c0 < w && c0 > 0) {
-        // avail: columns known to be published; q_{k+1} is read while q_k is
-        // applied when it is already there.
-        int avail = 0;
-        auto wait_for = [&](int k) {
-            while (avail <= k)
-                avail = __builtin_amdgcn_readfirstlane(
-                    __hip_atomic_load(&published, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP));
-        };
         float q[RPL], qn[RPL];
-        wait_for(0);
-        load_q(q, 0);
-        for (int k = 0; k < c0; ++k) {
-            const bool ahead = k + 1 < avail && k + 1 < c0;
-            if (ahead) load_q(qn, k + 1);
+        take(q, 0);
+        for (int k = 0; k + 1 < c0; ++k) {
+            const int n = peek(qn, k + 1);
             Acc d[kCPW];
-            project(q, std::integral_constant<int, 0>(), d);
+            project(q, d);
             if (lane == 0) {
 #pragma unroll
                 for (int c = 0; c < kCPW; ++c) Rs[k][c0 + c] = (float)d[c];
             }
-            if (!ahead && k + 1 < c0) {
-                wait_for(k + 1);
-                load_q(qn, k + 1);
-            }
+            if (__builtin_amdgcn_readfirstlane(n) <= k + 1) take(qn, k + 1);
 #pragma unroll
             for (int t = 0; t < RPL; ++t) q[t] = qn[t];
         }
+        __builtin_amdgcn_s_setprio(3);
+        Acc d[kCPW];
+        s0 = project_next(q, std::integral_constant<int, 0>(), d);
+        if (lane == 0) {
+#pragma unroll
+            for (int c = 0; c < kCPW; ++c) Rs[c0 - 1][c0 + c] = (float)d[c];
+        }
+    } else if (c0 == 0) {
+        Acc v[1] = {norm_terms(0)};
+        wave_sums(v);
+        s0 = v[0];
     }
     // This wave's own columns, ahead of the waves that only follow; R's
     // entries and Q are stored when the chain has left this wave.
     __builtin_amdgcn_s_setprio(3);
     Acc r[kCPW][kCPW];
     bool bad = false;
-    auto own = [&](auto col) {
+    auto own = [&](auto col, Acc s) -> Acc {
         constexpr int I = decltype(col)::value;
         const int k = c0 + I;
-        if (k >= w) return;
-        Acc s[1] = {(Acc)a[I][1] * (Acc)a[I][1]};
-        s[0] = fma((Acc)a[I][0], (Acc)a[I][0], s[0]);
-#pragma unroll
-        for (int t = 2; t < RPL; ++t) s[0] = fma((Acc)a[I][t], (Acc)a[I][t], s[0]);
-        wave_sums(s);
+        if (k >= w) return s;
         Acc nrm, inv;
-        const bool ok = norm_of(s[0], nrm, inv);
+        const bool ok = norm_of(s, nrm, inv);
         bad |= !ok;
         r[I][I] = ok ? nrm : (Acc)0;
 #pragma unroll
@@ -186,13 +240,14 @@ __device__ __forceinline__ void mgs_block_body(int m, int w, float *A, int64_t l
         // count sees q_k.
         asm volatile("" ::: "memory");
         if (lane == 0) __hip_atomic_store(&published, k + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-        if constexpr (I + 1 < kCPW) project(a[I], std::integral_constant<int, I + 1>(), r[I]);
+        if constexpr (I + 1 < kCPW) return project_next(a[I], std::integral_constant<int, I + 1>(), r[I]);
+        else return s;
     };
     static_assert(kCPW == 4, "four columns per wave");
-    own(std::integral_constant<int, 0>());
-    own(std::integral_constant<int, 1>());
-    own(std::integral_constant<int, 2>());
-    own(std::integral_constant<int, 3>());
+    const Acc s1 = own(std::integral_constant<int, 0>(), s0);
+    const Acc s2 = own(std::integral_constant<int, 1>(), s1);
+    const Acc s3 = own(std::integral_constant<int, 2>(), s2);
+    own(std::integral_constant<int, 3>(), s3);
     __builtin_amdgcn_s_setprio(0);
 #pragma unroll
     for (int i = 0; i < kCPW; ++i) {
