@@ -310,7 +310,7 @@ BATCH_BUCKETS = 56
 class BatchWg:
     """Batched QR of the column-major tensors As (in place) into Rs in one
     persistent kernel launch over a device work queue (later_batch_wg_*).
-    tuning: None (built-in table) or BATCH_BUCKETS variant ids."""
+    tuning: None (built-in table) or BATCH_BUCKETS variant ids (0 .. 4)."""
 
     def __init__(self, As, Rs, o: later_opts | None = None, tuning=None, status: bool = True):
         torch = _torch()

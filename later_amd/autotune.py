@@ -4,9 +4,10 @@ For every size bucket of the tuning table (later_batch_wg_bucket: n class
 min(ceil(n/32), 8) - 1, m class clamp(floor(log2 m) - 6, 0, 6)) it factors a
 synthetic batch of matrices drawn from that bucket (m log-uniform and n
 uniform inside the bucket's ranges, entries 2u - 1 from the Philox
-generator) with each variant of the kernel forced, and keeps the fastest:
-variant v runs panels of 16 << (v & 1) columns, projected against blocks of
-64 << (v >> 1) earlier columns of Q.  The batch of each bucket holds enough matrices for
+generator) with each variant forced, and keeps the fastest: variants 0 .. 3 run
+panels of 16 << (v & 1) columns, projected against blocks of 64 << (v >> 1)
+earlier columns of Q; variant 4 is the wide kernel (64-column panels against
+all earlier columns at once).  The batch of each bucket holds enough matrices for
 about 2e10 flops (64 to 2048 of them), timed as the minimum of three
 executions after one warm-up, on the mixed-form options.
 
@@ -23,7 +24,7 @@ import time
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 N_CLASSES, M_CLASSES = 8, 7
-VARIANTS = (0, 1, 2, 3)
+VARIANTS = (0, 1, 2, 3, 4)
 
 
 def bucket_ranges(nc: int, mc: int):
@@ -41,6 +42,7 @@ def tune(budget_flops: float = 2e10, log=print):
 
     o = L.opts("mixed")
     table = [-1] * (N_CLASSES * M_CLASSES)
+    narrow = [-1] * (N_CLASSES * M_CLASSES)  # the best of the variants 0 .. 3
     timings = {}
     for nc in range(N_CLASSES):
         for mc in range(M_CLASSES):
@@ -79,38 +81,43 @@ def tune(budget_flops: float = 2e10, log=print):
                 if best_ms is None or ms < best_ms:
                     best, best_ms = v, ms
             table[b] = best
+            narrow[b] = min((0, 1, 2, 3), key=lambda v: row[v])
             timings[b] = {"m": [m_lo, m_hi], "n": [n_lo, n_hi], "count": cnt, "ms": row, "best": best}
             log(f"[autotune] bucket {b:2d} m {m_lo}-{m_hi} n {n_lo}-{n_hi} ({cnt} matrices): "
                 + "  ".join(f"v{v} {row[v]:.3f} ms" for v in VARIANTS) + f"  -> v{best}")
             del As, A0, Rs
             torch.cuda.empty_cache()
-    return table, timings
+    return table, narrow, timings
 
 
-def write(table, timings, device: str):
+def write(table, narrow, timings, device: str):
     # Buckets with no shape keep the widest variant.
-    full = [3 if v < 0 else v for v in table]
-    lines = ["// Variant of the one-workgroup batched kernel per size bucket (see",
-             "// bucket_of): 0 = 16-column panels / 64-column blocks of earlier Q columns, 1 = 32 / 64,",
-             "// 2 = 16 / 128, 3 = 32 / 128.  Written by later_amd/autotune.py from",
-             f"// timings on {device}; rows are n classes (n <= 32, <= 64, ..., > 224),",
+    tables = {"kDefaultTuning": [4 if v < 0 else v for v in table],
+              "kNarrowTuning": [3 if v < 0 else v for v in narrow]}
+    lines = ["// Variant of the batched kernels per size bucket (see bucket_of): 0 = 16-column",
+             "// panels / 64-column blocks of earlier Q columns, 1 = 32 / 64, 2 = 16 / 128,",
+             "// 3 = 32 / 128, 4 = the wide kernel (kNarrowTuning: for 16-bit products and more",
+             "// than 256 columns, which it does not take).  Written by later_amd/autotune.py",
+             f"// from timings on {device}; rows are n classes (n <= 32, <= 64, ..., > 224),",
              "// columns m classes (m < 128, < 256, ..., >= 4096).",
-             "#pragma once",
-             "constexpr int kDefaultTuning[kBuckets] = {"]
-    for nc in range(N_CLASSES):
-        lines.append("    " + ", ".join(str(full[M_CLASSES * nc + mc]) for mc in range(M_CLASSES)) + ",")
-    lines.append("};")
+             "#pragma once"]
+    for name, full in tables.items():
+        lines.append(f"constexpr int {name}[kBuckets] = {{")
+        for nc in range(N_CLASSES):
+            lines.append("    " + ", ".join(str(full[M_CLASSES * nc + mc]) for mc in range(M_CLASSES)) + ",")
+        lines.append("};")
     with open(os.path.join(HERE, "csrc", "batch_tuning.h"), "w") as f:
         f.write("\n".join(lines) + "\n")
     with open(os.path.join(HERE, "batch_tuning.json"), "w") as f:
-        json.dump({"device": device, "table": full, "buckets": timings}, f, indent=1, sort_keys=True)
+        json.dump({"device": device, "table": tables["kDefaultTuning"], "narrow": tables["kNarrowTuning"],
+                   "buckets": timings}, f, indent=1, sort_keys=True)
 
 
 def main():
     import torch
     t0 = time.time()
-    table, timings = tune(log=lambda *a: print(*a, flush=True))
-    write(table, timings, torch.cuda.get_device_name(0) + " (gfx950)")
+    table, narrow, timings = tune(log=lambda *a: print(*a, flush=True))
+    write(table, narrow, timings, torch.cuda.get_device_name(0) + " (gfx950)")
     print(f"[autotune] done in {time.time() - t0:.1f} s", flush=True)
 
 

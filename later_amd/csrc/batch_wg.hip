@@ -1,5 +1,8 @@
 // Batched QR in one persistent launch: every workgroup takes whole matrices
-// from a device work queue and factors each one by itself.
+// from a device work queue and factors each one by itself.  This file holds
+// the queue, the plan and the kernel for 16-bit products, narrow matrices and
+// more than 256 columns; FP32 products of 33 .. 256 columns run
+// batch_wide.hip's.
 //
 // The queue is the task table, ordered by size bucket and, inside a bucket,
 // by decreasing cost (largest matrices first, so the long tasks start
@@ -31,6 +34,7 @@
 
 #include <type_traits>
 
+#include "batch_wg.h"
 #include "chol_dev.h"
 #include "common.h"
 
@@ -39,19 +43,6 @@ namespace {
 constexpr int kKC = 64;            // rows per staged chunk
 constexpr int kLDC = kKC + 1;      // stride of a column-major LDS chunk (odd: conflict-free)
 constexpr int kNTBMax = 128;       // earlier Q columns per block (max)
-
-struct WgTask {
-    int m, n, variant, pad;
-    float *A;
-    int64_t lda;
-    float *R;
-    int64_t ldr;
-    int *status;
-};
-
-struct WgQueue {
-    unsigned int head, done;
-};
 
 // Variant v: panel width 16 << (v & 1), blocks of 64 << (v >> 1) earlier Q columns.
 __host__ __device__ constexpr int variant_bw(int v) { return 16 << (v & 1); }
@@ -540,12 +531,8 @@ template <int PREC>
 __global__ __launch_bounds__(kThreads, 2) void batch_wg_kernel(const WgTask *tasks, int ntasks, WgQueue *q, int reorth)
 {
     __shared__ __attribute__((aligned(16))) char lds[WgLds::kBytes];
-    __shared__ unsigned int cur;
     for (;;) {
-        if (threadIdx.x == 0) cur = atomicAdd(&q->head, 1u);
-        __syncthreads();
-        const unsigned int t = cur;
-        __syncthreads();
+        const unsigned int t = wg_next_task(q);
         if (t >= (unsigned int)ntasks) break;
         const WgTask tk = tasks[t];
         if (threadIdx.x == 0 && tk.status) *tk.status = 0;
@@ -558,13 +545,7 @@ __global__ __launch_bounds__(kThreads, 2) void batch_wg_kernel(const WgTask *tas
         }
         __syncthreads();
     }
-    if (threadIdx.x == 0) {
-        const unsigned int d = atomicAdd(&q->done, 1u);
-        if (d == gridDim.x - 1) {
-            atomicExch(&q->head, 0u);
-            atomicExch(&q->done, 0u);
-        }
-    }
+    wg_leave(q);
 }
 
 } // namespace
@@ -597,12 +578,16 @@ int wg_prec(const later_opts &o)
     }
 }
 
+// Tasks 0 .. nwide - 1 run on the wide kernel (variant 4), the rest on the
+// narrow one; each kernel has its own queue.
 struct WgPlan {
     void *dev = nullptr;
     WgTask *tasks = nullptr;
     WgQueue *q = nullptr;
-    int ntasks = 0, grid = 0, prec = 0, reorth = 0;
+    int ntasks = 0, nwide = 0, grid = 0, grid_wide = 0, prec = 0, reorth = 0;
 };
+
+constexpr int kWideVariant = 4;
 
 } // namespace
 
@@ -618,28 +603,44 @@ LATER_API int later_batch_wg_create(int count, const int *m, const int *n, float
     if (o.gemm < LATER_GEMM_F32 || o.gemm > LATER_GEMM_I8X4 || o.reorth < 0 || o.reorth > 3) return LATER_ERR_OPTION;
     std::vector<WgTask> tasks(count);
     std::vector<std::pair<double, int>> order(count);
+    const bool f32 = wg_prec(o) == LATER_GEMM_F32;
+    double work_narrow = 0.0, work_wide = 0.0;  // of the tasks by the table, in columns x rows of the wide kernel's sweeps
     for (int i = 0; i < count; ++i) {
         if (m[i] < 1 || n[i] < 1 || m[i] < n[i] || lda[i] < m[i] || ldr[i] < n[i] || !A[i] || !R[i])
             return LATER_ERR_SHAPE;
         const int b = bucket_of(m[i], n[i]);
         int v = tuning ? tuning[b] : kDefaultTuning[b];
-        if (v < 0 || v > 3) v = kDefaultTuning[b];
+        if (v < 0 || v > kWideVariant) v = kDefaultTuning[b];
+        if (v == kWideVariant && !(f32 && n[i] <= kWideCols && m[i] >= 4)) v = kNarrowTuning[b];
+        (v == kWideVariant ? work_wide : work_narrow) += 4.0 * m[i] * std::max(64, n[i]) * (double)std::max(64, n[i]);
         tasks[i] = WgTask{m[i], n[i], v, 0, A[i], (int64_t)lda[i], R[i], (int64_t)ldr[i], status ? status + i : nullptr};
+    }
+    // The two kernels run one after the other, so a small share of tasks that
+    // the narrow one would do faster by itself (up to a quarter of the work)
+    // fills the wide one's last wave instead of adding a launch.
+    const bool join = !tuning && f32 && work_narrow <= 0.25 * work_wide;
+    for (int i = 0; i < count; ++i) {
+        if (join && n[i] <= kWideCols && m[i] >= 4) tasks[i].variant = kWideVariant;
+        const int v = tasks[i].variant;
         // Cost: the products (4 m n^2 with the second projection) plus the
         // sequential panel factorisations (~ n / BW Cholesky factors).
-        const double cost = 4.0 * m[i] * (double)n[i] * n[i] + 2.0e6 * ((n[i] + variant_bw(v) - 1) / variant_bw(v));
+        const int bw = v == kWideVariant ? 64 : variant_bw(v);
+        const double cost = 4.0 * m[i] * (double)n[i] * n[i] + 2.0e6 * ((n[i] + bw - 1) / bw);
         order[i] = {-cost, i};
     }
     std::stable_sort(order.begin(), order.end());
+    const auto split = std::stable_partition(order.begin(), order.end(), [&](const std::pair<double, int> &x) {
+        return tasks[x.second].variant == kWideVariant;
+    });
     std::vector<WgTask> sorted(count);
     for (int i = 0; i < count; ++i) sorted[i] = tasks[order[i].second];
     WgPlan *P = new WgPlan();
     const size_t tbytes = ((size_t)count * sizeof(WgTask) + 255) / 256 * 256;
-    if (hipMalloc(&P->dev, tbytes + 256) != hipSuccess) { delete P; return LATER_ERR_DEVICE; }
+    if (hipMalloc(&P->dev, tbytes + 2 * sizeof(WgQueue)) != hipSuccess) { delete P; return LATER_ERR_DEVICE; }
     P->tasks = (WgTask *)P->dev;
     P->q = (WgQueue *)((char *)P->dev + tbytes);
     if (hipMemcpy(P->tasks, sorted.data(), (size_t)count * sizeof(WgTask), hipMemcpyHostToDevice) != hipSuccess ||
-        hipMemset(P->q, 0, sizeof(WgQueue)) != hipSuccess) {
+        hipMemset(P->q, 0, 2 * sizeof(WgQueue)) != hipSuccess) {
         hipFree(P->dev);
         delete P;
         return LATER_ERR_DEVICE;
@@ -652,7 +653,10 @@ LATER_API int later_batch_wg_create(int count, const int *m, const int *n, float
     }
     // Two workgroups per CU (the kernel's LDS allows two).
     P->ntasks = count;
-    P->grid = count < 2 * cus ? count : 2 * cus;
+    P->nwide = (int)(split - order.begin());
+    const int narrow = count - P->nwide;
+    P->grid = narrow < 2 * cus ? narrow : 2 * cus;
+    P->grid_wide = P->nwide < cus ? P->nwide : cus;
     P->prec = wg_prec(o);
     P->reorth = o.reorth != 0 ? 1 : 0;
     *plan = P;
@@ -664,18 +668,26 @@ LATER_API int later_batch_wg_execute(void *plan, void *stream)
     WgPlan *P = (WgPlan *)plan;
     if (!P || !P->dev) return LATER_ERR_SHAPE;
     hipStream_t s = (hipStream_t)stream;
+    if (P->nwide > 0) {
+        const int rc = batch_wide_launch(s, P->tasks, P->nwide, P->q, P->grid_wide, P->reorth != 0);
+        if (rc) return rc;
+    }
+    const int narrow = P->ntasks - P->nwide;
+    if (narrow == 0) return LATER_OK;
+    const WgTask *t = P->tasks + P->nwide;
+    WgQueue *q = P->q + 1;
     switch (P->prec) {
     case LATER_GEMM_F16:
-        hipLaunchKernelGGL(batch_wg_kernel<LATER_GEMM_F16>, dim3(P->grid), dim3(kThreads), 0, s, P->tasks, P->ntasks,
-                           P->q, P->reorth);
+        hipLaunchKernelGGL(batch_wg_kernel<LATER_GEMM_F16>, dim3(P->grid), dim3(kThreads), 0, s, t, narrow, q,
+                           P->reorth);
         break;
     case LATER_GEMM_BF16:
-        hipLaunchKernelGGL(batch_wg_kernel<LATER_GEMM_BF16>, dim3(P->grid), dim3(kThreads), 0, s, P->tasks,
-                           P->ntasks, P->q, P->reorth);
+        hipLaunchKernelGGL(batch_wg_kernel<LATER_GEMM_BF16>, dim3(P->grid), dim3(kThreads), 0, s, t, narrow, q,
+                           P->reorth);
         break;
     default:
-        hipLaunchKernelGGL(batch_wg_kernel<LATER_GEMM_F32>, dim3(P->grid), dim3(kThreads), 0, s, P->tasks, P->ntasks,
-                           P->q, P->reorth);
+        hipLaunchKernelGGL(batch_wg_kernel<LATER_GEMM_F32>, dim3(P->grid), dim3(kThreads), 0, s, t, narrow, q,
+                           P->reorth);
         break;
     }
     HIP_OK(hipGetLastError());

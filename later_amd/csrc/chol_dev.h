@@ -298,16 +298,18 @@ __device__ __forceinline__ bool eliminate16_wave(const double *S, const double *
 // end.  Wave 0 updates the next diagonal block and goes on to its
 // elimination while the other waves update the rest, so the serial path is
 // the W / 16 eliminations and one product before and after each.  A pivot is
-// compared with the diagonal of G.  Destroys Gs.  Called by every thread of
-// the workgroup; returns (on wave 0) whether a pivot was bad.
+// compared with the diagonal of G.  Destroys Gs.  nb: the blocks to factor
+// (the columns behind them are left undefined).  Called by every thread of the
+// workgroup (four waves or more); returns (on wave 0) whether a pivot was bad.
 // Bound: the dependent FP64 chain of the pivots (about 100 cycles each) and
 // the issue of the rank-1 rows beside it.  W = 64: 10 us, where two 32 x 32
 // one-wave eliminations, fully unrolled with scalar broadcasts and each
 // pivot's square root on the chain, took 19 us (a first-pass leaf of 8192 x 64:
 // factor and apply 30 -> 21 us).
-template <int W> __device__ __forceinline__ bool factor(double *Gs, double *Rs, double *Ris, double *d0)
+template <int W>
+__device__ __forceinline__ bool factor(double *Gs, double *Rs, double *Ris, double *d0, int nb = W / 16)
 {
-    constexpr int LDG = Shape<W>::LDG, NB = W / 16;
+    constexpr int LDG = Shape<W>::LDG;
     const int t = threadIdx.x, lane = t & 63, wv = __builtin_amdgcn_readfirstlane(t >> 6);
     const int li = lane & 15, lk = lane >> 4;
     double *U = Ris, *M = Ris + 256, *isq = Ris + 256 + 16 * kLdM;
@@ -349,16 +351,16 @@ template <int W> __device__ __forceinline__ bool factor(double *Gs, double *Rs, 
     };
     bool bad = false;
 #pragma unroll 1
-    for (int b = 0; b < NB; ++b) {
+    for (int b = 0; b < nb; ++b) {
         if (wv == 0) {
             if (b > 0) trailing(b - 1, b, b);
             bad |= eliminate16_wave<LDG>(Gs + 16 * b * LDG + 16 * b, d0 + 16 * b, U, M, isq);
         } else if (b > 0) {
             int n = 0;
 #pragma unroll 1
-            for (int i = b; i < NB; ++i)
+            for (int i = b; i < nb; ++i)
 #pragma unroll 1
-                for (int j = 0; j < NB; ++j)
+                for (int j = 0; j < nb; ++j)
                     if ((i <= j || j < b) && !(i == b && j == b)) {
                         if (n == wv - 1) trailing(b - 1, i, j);
                         n = n == 2 ? 0 : n + 1;
@@ -374,10 +376,10 @@ template <int W> __device__ __forceinline__ bool factor(double *Gs, double *Rs, 
                 Rs[(16 * b + k) * W + 16 * b + li] = li < k ? 0.0 : U[k * 16 + li] * s;
                 Gs[(16 * b + k) * LDG + 16 * b + li] = M[k * kLdM + li] * s;
             }
-        } else if (wv < NB - 1) {
-            // Row b of R and of X: block j on wave (j - b - 1) mod NB, so that
+        } else if (wv < nb - 1) {
+            // Row b of R and of X: block j on wave (j - b - 1) mod nb, so that
             // the next diagonal block's factor R_b,b+1 is wave 0's.
-            const int j = (b + 1 + wv) % NB;
+            const int j = (b + 1 + wv) % nb;
             double av[4];
 #pragma unroll
             for (int s = 0; s < 4; ++s) av[s] = M[li * kLdM + 4 * s + lk] * isq[li];
