@@ -40,6 +40,8 @@
 
 namespace {
 
+typedef float floatx4u __attribute__((ext_vector_type(4), aligned(4)));  // one dwordx4 load at any dword address
+
 // Sum of more than kDirect partial Grams, in a fixed tree: workgroup b owns
 // entries 32b .. 32b+31; thread (q, e) adds groups q*G/8 .. (q+1)*G/8 - 1 in
 // order, then the eight part sums are added in order of q.
@@ -93,6 +95,16 @@ template <int W> struct BlockRegs {
             }
         }
     }
+    // All W columns of 64 rows that all lie inside the panel, at any dword
+    // alignment and without a branch (a branch around a load makes the
+    // compiler wait at the join for every load in flight).
+    __device__ __forceinline__ void load_inside(const float *A, int64_t lda, int r0)
+    {
+        const int t = threadIdx.x;
+#pragma unroll
+        for (int j = 0; j < NV; ++j)
+            v[j] = *(const floatx4u *)(A + (int64_t)((t >> 4) + 16 * j) * lda + r0 + 4 * (t & 15));
+    }
     __device__ __forceinline__ void store_ld(float *Qs, int ld) const
     {
         const int t = threadIdx.x;
@@ -103,9 +115,15 @@ template <int W> struct BlockRegs {
     __device__ __forceinline__ void store(float *Qs) const { store_ld(Qs, kRows + 4); }
 };
 
+// The last of the 64-row blocks 0, 1, .. that lie inside a panel of full
+// width (-1: none).
+__device__ __forceinline__ int inside_last(int m, int w, int W) { return w == W ? m / kRows - 1 : -1; }
+
 // Partial Gram of the rows of this workgroup (64-row blocks b, b + G, ...)
 // into p1[blockIdx.x]: coalesced loads two blocks ahead, the block staged in
-// LDS, FP64 MFMA per 16-row group of each wave.
+// LDS, FP64 MFMA per 16-row group of each wave.  Bound by FP64 MFMA (68 us for
+// 1048576 x 64); with the loads of blocks inside the panel free of branches
+// they are two blocks ahead in fact: 136 -> 105 us.
 template <int W>
 __global__ __launch_bounds__(kThreads) void chol_gram_kernel(int m, int w, const float *A, int64_t lda, float *ws)
 {
@@ -118,20 +136,42 @@ __global__ __launch_bounds__(kThreads) void chol_gram_kernel(int m, int w, const
     const int wv = threadIdx.x >> 6;
     Gram<W> g;
     gram_zero<W>(g);
-    BlockRegs<W> r[2];
-    int b = blockIdx.x;
-    if (b < nblk) r[0].load(A, lda, m, w, b * kRows);
-    if (b + G < nblk) r[1].load(A, lda, m, w, (b + G) * kRows);
-    for (int it = 0; b < nblk; b += G, ++it) {
+    BlockRegs<W> r0, r1;
+    auto block = [&](const BlockRegs<W> &r) {
         __syncthreads();  // the previous block has been read
-        if (it & 1) r[1].store(Qs); else r[0].store(Qs);
+        r.store(Qs);
         __syncthreads();
-        if (b + 2 * G < nblk) {
-            if (it & 1) r[1].load(A, lda, m, w, (b + 2 * G) * kRows);
-            else r[0].load(A, lda, m, w, (b + 2 * G) * kRows);
-        }
+    };
+    auto product = [&]() {
 #pragma unroll
         for (int sg = 0; sg < kTT; ++sg) gram_lds<W>(g, Qs, (wv * kTT + sg) * 16);
+    };
+    int b = blockIdx.x;
+    const int last = inside_last(m, w, W);  // blocks up to here need no test
+    if (b + 3 * G <= last) {
+        r0.load_inside(A, lda, b * kRows);
+        __builtin_amdgcn_sched_barrier(0);  // r0 first: the loop's waits count on the order
+        r1.load_inside(A, lda, (b + G) * kRows);
+#pragma unroll 1
+        for (; b + 3 * G <= last; b += 2 * G) {
+            block(r0);
+            r0.load_inside(A, lda, (b + 2 * G) * kRows);
+            product();
+            block(r1);
+            r1.load_inside(A, lda, (b + 3 * G) * kRows);
+            product();
+        }
+    } else {
+        if (b < nblk) r0.load(A, lda, m, w, b * kRows);
+        if (b + G < nblk) r1.load(A, lda, m, w, (b + G) * kRows);
+    }
+    for (int it = 0; b < nblk; b += G, ++it) {
+        if (it & 1) block(r1); else block(r0);
+        if (b + 2 * G < nblk) {
+            if (it & 1) r1.load(A, lda, m, w, (b + 2 * G) * kRows);
+            else r0.load(A, lda, m, w, (b + 2 * G) * kRows);
+        }
+        product();
     }
     __syncthreads();
     gram_finish<W>(g, (double *)smem, cw.p1 + (int64_t)blockIdx.x * Shape<W>::P);
@@ -214,7 +254,8 @@ __global__ __launch_bounds__(kThreads) void chol_factor_kernel(int w, float *ws,
 // (up to four independent MFMAs in flight); D's lanes walk 16 consecutive
 // rows of one column (64-byte stores).  PASS 1 also forms the partial Gram
 // of the stored Q1 rows into p2[blockIdx.x] (then the grid is the Gram
-// kernel's).
+// kernel's).  Bound by memory (110 us for 1048576 x 64 at a copy's rate);
+// without a branch around a load or a store it takes 127 us, 152 before.
 constexpr int kApplyLd = kRows + 16;
 
 template <int PASS, int W>
@@ -233,10 +274,8 @@ __global__ __launch_bounds__(kThreads) void chol_apply_kernel(int m, int w, floa
     const int G = gridDim.x;
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
 
-    BlockRegs<W> r[2];
+    BlockRegs<W> r0, r1;
     int b = blockIdx.x;
-    if (b < nblk) r[0].load(A, lda, m, w, b * kRows);
-    if (b + G < nblk) r[1].load(A, lda, m, w, (b + G) * kRows);
     // A-operand slices of R^{-1}: rv[ct][s] = R^{-1}[4 s + l/16][16 ct + l%16]
     // (zero for k > column, so column tile ct needs k-steps 0 .. 4 ct + 3).
     double rv[CT][KS];
@@ -248,15 +287,13 @@ __global__ __launch_bounds__(kThreads) void chol_apply_kernel(int m, int w, floa
 
     Gram<W> g;
     if constexpr (PASS == 1) gram_zero<W>(g);
-#pragma unroll 1
-    for (int it = 0; b < nblk; b += G, ++it) {
+    auto block = [&](const BlockRegs<W> &r) {
         __syncthreads();  // the previous block's operands have been read
-        if (it & 1) r[1].store_ld(As, kApplyLd); else r[0].store_ld(As, kApplyLd);
+        r.store_ld(As, kApplyLd);
         __syncthreads();
-        if (b + 2 * G < nblk) {
-            if (it & 1) r[1].load(A, lda, m, w, (b + 2 * G) * kRows);
-            else r[0].load(A, lda, m, w, (b + 2 * G) * kRows);
-        }
+    };
+    // Q of the staged block b (inside: its rows and columns all exist).
+    auto product = [&](int b, auto inside) {
         const int lrow = wv * 16 + (lane & 15);  // row within the block
         const int row = b * kRows + lrow;
         float av[KS];
@@ -276,7 +313,7 @@ __global__ __launch_bounds__(kThreads) void chol_apply_kernel(int m, int w, floa
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
                 const int col = 16 * ct + (lane >> 4) + 4 * q;
-                const bool ok = row < m && col < w;
+                const bool ok = decltype(inside)::value || (row < m && col < w);
                 const float v = ok ? (float)d[ct][q] : 0.0f;
                 if (ok) A[row + (int64_t)col * lda] = v;
                 if constexpr (PASS == 1) Qs[col * (kRows + 4) + lrow] = v;
@@ -287,6 +324,39 @@ __global__ __launch_bounds__(kThreads) void chol_apply_kernel(int m, int w, floa
 #pragma unroll
             for (int sg = 0; sg < kTT; ++sg) gram_lds<W>(g, Qs, (wv * kTT + sg) * 16);
         }
+    };
+    const int last = inside_last(m, w, W);
+    if (b + 3 * G <= last) {
+        r0.load_inside(A, lda, b * kRows);
+        __builtin_amdgcn_sched_barrier(0);  // r0 first: the loop's waits count on the order
+        r1.load_inside(A, lda, (b + G) * kRows);
+        auto pair = [&]() {
+            block(r0);
+            r0.load_inside(A, lda, (b + 2 * G) * kRows);
+            product(b, std::true_type());
+            block(r1);
+            r1.load_inside(A, lda, (b + 3 * G) * kRows);
+            product(b + G, std::true_type());
+            b += 2 * G;
+        };
+        // The first pair stands apart: the loop's waits are set by the path
+        // with the fewest requests behind a block's loads, and before the
+        // first pair no stores are.
+        pair();
+#pragma unroll 1
+        while (b + 3 * G <= last) pair();
+    } else {
+        if (b < nblk) r0.load(A, lda, m, w, b * kRows);
+        if (b + G < nblk) r1.load(A, lda, m, w, (b + G) * kRows);
+    }
+#pragma unroll 1
+    for (int it = 0; b < nblk; b += G, ++it) {
+        if (it & 1) block(r1); else block(r0);
+        if (b + 2 * G < nblk) {
+            if (it & 1) r1.load(A, lda, m, w, (b + 2 * G) * kRows);
+            else r0.load(A, lda, m, w, (b + 2 * G) * kRows);
+        }
+        product(b, std::false_type());
     }
     if constexpr (PASS == 1) {
         __syncthreads();

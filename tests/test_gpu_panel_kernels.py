@@ -112,3 +112,46 @@ def test_trsm_upper_blocks(later, oracle, n, k, zero):
     R = R.astype(np.float64)
     res = np.abs(R @ X - B)[rows]
     assert np.all(res <= (2.0 ** -24 + n * 2.0 ** -50) * (np.abs(R) @ np.abs(X))[rows] + 1e-30)
+
+
+# Products whose operands are converted on the way to LDS: slab counts around
+# the untested loop's start, ragged K, tile rows and columns, leading dimension
+# and address at any dword (K-major both, then rows of A along M).  An element
+# is a chain of K fused products (and a few FP64 sums) of operands kept to 24
+# (F32, F16X6), 22 (F16X3) or 11 bits (F16): K + 2 units of 2^-24 of its terms'
+# magnitudes, 16 more for the dropped low pieces, 2^-10 for one piece.
+@pytest.mark.parametrize("k", [128, 129, 160, 161, 321, 575, 640, 1089])
+@pytest.mark.parametrize("n1,n2,pad", [(64, 192, 0), (131, 129, 1), (300, 257, 3)])
+@pytest.mark.parametrize("prec,extra", [("GEMM_F32", 0.0), ("GEMM_F16X6", 16.0), ("GEMM_F16X3", 16.0),
+                                        ("GEMM_F16", 2.0 ** 14)])
+def test_staged_products(later, oracle, k, n1, n2, pad, prec, extra):
+    u, p = 2.0 ** -24, getattr(later, prec)
+    A, B = oracle.gen_uniform(k, n1, 1, 1), oracle.gen_uniform(k, n2, 2, 2)
+    a, b = _dev(later, A, pad), _dev(later, B, pad)
+    P = _np(later.gemm_proj(a, b, later.colmajor(n1, n2, ld=n1 + pad), p))
+    A, B = A.astype(np.float64), B.astype(np.float64)
+    assert np.all(np.abs(P - A.T @ B) <= (k + 2 + extra) * u * (np.abs(A).T @ np.abs(B)) + k * 2.0 ** -22 * (extra > 16))
+    Q, C, D = oracle.gen_uniform(n1, k, 3, 3), oracle.gen_uniform(k, n2, 4, 4), oracle.gen_uniform(n1, n2, 5, 5)
+    q, c, d = _dev(later, Q, pad), _dev(later, C, pad), _dev(later, D, pad)
+    U = _np(later.gemm_update(q, c, d, p))
+    Q, C, D = (x.astype(np.float64) for x in (Q, C, D))
+    assert np.all(np.abs(U - (D - Q @ C)) <= (k + 2 + extra) * u * (np.abs(Q) @ np.abs(C)) + 2 * u * np.abs(D)
+                  + k * 2.0 ** -22 * (extra > 16))
+
+
+# Tall Cholesky leaves: four blocks and more for some workgroups of the grid
+# (512 blocks of 64 rows are one each), a ragged last block, widths short of
+# the kernel's, odd leading dimensions.  FP64 Grams and two passes: Q within
+# the FP32 rounding of its entries.
+@pytest.mark.parametrize("m", [98304, 131072 + 64 * 5 + 17, 262144 + 3])
+@pytest.mark.parametrize("w,pad", [(64, 0), (64, 1), (63, 3), (32, 1), (20, 0)])
+def test_tall_cholesky_leaf(later, oracle, m, w, pad):
+    A = oracle.gen_uniform(m, w, 9, 4)
+    X = _dev(later, A, pad)
+    o = later.opts("mixed")
+    work = later.workspace(m, w, o)
+    R = later.rgsqrf(X, o=o, work=work)
+    torch.cuda.synchronize()
+    Q, R = _np(X), _np(R)
+    assert later.read_status(work) == 0
+    assert oracle.orth(Q) < 2e-6 * np.sqrt(w) and oracle.backward(A, Q, R) < 1e-6
