@@ -341,9 +341,81 @@ __device__ __forceinline__ typename Frag<PREC>::T frag(const typename Lds<PREC>:
 // and columns 8 (r/4) + 4 (l/32) + r%4, r = 0..15.
 // ROWEXP: rows of op(A) carry their own exponents (int8 slices, at byte
 // offset lsa from Ah); the result is scaled by 2^-(a_exp + row's + column's).
+//
+// store_tile_inside: the same for a wave tile that lies inside C, 32 x 32
+// block by block.  A block's exponents and, for an update, its C values are
+// requested together, while the block before is stored, and nothing is tested
+// per element; the general form takes one load of an exponent, one wait and
+// one branch per element (mixed 8192 x 1024 1.87 -> 1.75 ms, 262144 x 256 with
+// FP8 projections 2.17 -> 1.86 ms, FP32 8192 x 4096 9.9 -> 9.7 ms).
+template <bool CH64, int FM, int FN, typename V, bool ROWEXP>
+__device__ __forceinline__ void store_tile_inside(const GemmArgs &g, int split, int row0, int col0, V value)
+{
+    typedef int intx4u __attribute__((ext_vector_type(4), aligned(4)));
+    const int lane = threadIdx.x & 63;
+    const int row = row0 + (lane & 31), col = col0 + 4 * (lane >> 5);
+    const bool rmw = !g.partial && g.update;
+    struct Block {
+        int e[16];     // exponents, a column's and the row's
+        float c[16];   // C, for an update
+    };
+    auto *c = gmem(g.C) + (int64_t)col * g.ldc + row;
+    auto col_of = [](int r) { return 8 * (r >> 2) + (r & 3); };  // less the block's and the lane's
+    auto load = [&](Block &b, int i, int j) {
+        const int re = g.a_exp + (ROWEXP ? gmem((const int *)((const char *)g.Ah + g.lsa))[row + 32 * i] : 0);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            intx4u x = {0, 0, 0, 0};
+            if (g.b_exp) x = *(const __attribute__((address_space(1))) intx4u *)(gmem(g.b_exp) + col + 32 * j + 8 * q);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) b.e[4 * q + r] = re + x[r];
+        }
+        if (rmw)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) b.c[r] = c[(int64_t)(32 * j + col_of(r)) * g.ldc + 32 * i];
+    };
+    Block b[2];
+    constexpr bool kAhead = !ROWEXP;  // int8 groups leave no registers for a second block
+    if (kAhead) load(b[0], 0, 0);
+#pragma unroll
+    for (int n = 0; n < FM * FN; ++n) {
+        const int i = n / FN, j = n % FN;
+        if (!kAhead) load(b[n & 1], i, j);
+        if (kAhead && n + 1 < FM * FN) load(b[(n + 1) & 1], (n + 1) / FN, (n + 1) % FN);
+        const Block &k = b[n & 1];
+        auto scaled = [&](int r) -> double { return value(i, j, r) * ldexp(1.0, -k.e[r]); };
+        if (rmw && (CH64 || g.update == 2)) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r)
+                c[(int64_t)(32 * j + col_of(r)) * g.ldc + 32 * i] =
+                    (float)((double)k.c[r] + (double)g.alpha * scaled(r));
+        } else if (rmw) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r)
+                c[(int64_t)(32 * j + col_of(r)) * g.ldc + 32 * i] = fmaf(g.alpha, (float)scaled(r), k.c[r]);
+        } else if (!g.partial) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) c[(int64_t)(32 * j + col_of(r)) * g.ldc + 32 * i] = (float)scaled(r);
+        } else {
+            const int64_t off = ((int64_t)split * g.N + col + 32 * j) * g.M + row + 32 * i;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                if constexpr (CH64) gmem((double *)g.partial)[off + (int64_t)col_of(r) * g.M] = scaled(r);
+                else gmem((float *)g.partial)[off + (int64_t)col_of(r) * g.M] = (float)scaled(r);
+            }
+        }
+    }
+}
+
 template <bool CH64, int FM, int FN, typename V, bool ROWEXP = false>
 __device__ __forceinline__ void store_tile(const GemmArgs &g, int split, int row0, int col0, V value)
 {
+    row0 = __builtin_amdgcn_readfirstlane(row0);
+    col0 = __builtin_amdgcn_readfirstlane(col0);
+    if (row0 + 32 * FM <= g.M && col0 + 32 * FN <= g.N) {
+        store_tile_inside<CH64, FM, FN, V, ROWEXP>(g, split, row0, col0, value);
+        return;
+    }
     const int lane = threadIdx.x & 63;
     const bool rmw = !g.partial && g.update;
 #pragma unroll

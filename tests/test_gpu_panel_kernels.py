@@ -155,3 +155,21 @@ def test_tall_cholesky_leaf(later, oracle, m, w, pad):
     Q, R = _np(X), _np(R)
     assert later.read_status(work) == 0
     assert oracle.orth(Q) < 2e-6 * np.sqrt(w) and oracle.backward(A, Q, R) < 1e-6
+
+
+# Streamed products of pre-split operands: wave tiles inside C and at its edges
+# (64 and 32 rows of a wave), exponents of B at any dword address, an update and
+# a projection with and without splits.  Bounds as above.
+@pytest.mark.parametrize("m,n1,n2", [(512, 192, 160), (3000, 257, 130), (1100, 320, 97)])
+@pytest.mark.parametrize("pad", [0, 1])
+@pytest.mark.parametrize("prec,extra", [("GEMM_F16X6", 16.0), ("GEMM_F16X3", 16.0), ("GEMM_F16", 2.0 ** 14)])
+def test_streamed_products(later, oracle, m, n1, n2, pad, prec, extra):
+    u, p = 2.0 ** -24, getattr(later, prec)
+    Q, B, C = oracle.gen_uniform(m, n1, 1, 1), oracle.gen_uniform(m, n2, 2, 2), oracle.gen_uniform(n1, n2, 3, 3)
+    q, b, c = _dev(later, Q, pad), _dev(later, B, pad), _dev(later, C, pad)
+    P = _np(later.gemm_proj(q, b, later.colmajor(n1, n2, ld=n1 + pad), p, pieces=True))
+    U = _np(later.gemm_update(q, c, b, p, pieces=True))
+    Q, B, C = (x.astype(np.float64) for x in (Q, B, C))
+    assert np.all(np.abs(P - Q.T @ B) <= (m + 2 + extra) * u * (np.abs(Q).T @ np.abs(B)) + m * 2.0 ** -22 * (extra > 16))
+    assert np.all(np.abs(U - (B - Q @ C)) <= (n1 + 2 + extra) * u * (np.abs(Q) @ np.abs(C)) + 2 * u * np.abs(B)
+                  + n1 * 2.0 ** -22 * (extra > 16))
