@@ -44,8 +44,10 @@ typedef float floatx4u __attribute__((ext_vector_type(4), aligned(4)));  // one 
 
 // Sum of more than kDirect partial Grams, in a fixed tree: workgroup b owns
 // entries 32b .. 32b+31; thread (q, e) adds groups q*G/8 .. (q+1)*G/8 - 1 in
-// order, then the eight part sums are added in order of q.
-template <int W> __global__ __launch_bounds__(256) void chol_reduce_kernel(const double *part, int ngroups, double *out)
+// order, then the eight part sums are added in order of q.  The result is
+// stored as the full matrix, so that no reader has to unpack it.
+template <int W>
+__global__ __launch_bounds__(256) void chol_reduce_kernel(const double *part, int ngroups, int w, double *out)
 {
     __shared__ double ps[8][32];
     const int e = blockIdx.x * 32 + (threadIdx.x & 31), q = threadIdx.x >> 5;
@@ -68,7 +70,11 @@ template <int W> __global__ __launch_bounds__(256) void chol_reduce_kernel(const
         double t = ps[0][threadIdx.x];
 #pragma unroll
         for (int k = 1; k < 8; ++k) t += ps[k][threadIdx.x];
-        out[e] = t;
+        int i, j;
+        unpack(e, i, j);
+        if (i >= w || j >= w) t = (i == j) ? 1.0 : 0.0;
+        out[i * W + j] = t;
+        out[j * W + i] = t;
     }
 }
 
@@ -127,7 +133,7 @@ __device__ __forceinline__ int inside_last(int m, int w, int W) { return w == W 
 template <int W>
 __global__ __launch_bounds__(kThreads) void chol_gram_kernel(int m, int w, const float *A, int64_t lda, float *ws)
 {
-    constexpr int kQs = W * (kRows + 4) * 4, kCb = 2 * Shape<W>::NT * 4 * 64 * 8;
+    constexpr int kQs = W * (kRows + 4) * 4, kCb = kGramLds<W>;
     __shared__ __attribute__((aligned(16))) char smem[kQs > kCb ? kQs : kCb];
     float *Qs = (float *)smem;
     const CholWork cw = carve<W>(ws);
@@ -174,7 +180,7 @@ __global__ __launch_bounds__(kThreads) void chol_gram_kernel(int m, int w, const
         product();
     }
     __syncthreads();
-    gram_finish<W>(g, (double *)smem, cw.p1 + (int64_t)blockIdx.x * Shape<W>::P);
+    gram_finish_shared<W>(g, (double *)smem, cw.p1 + (int64_t)blockIdx.x * Shape<W>::P);
 }
 
 // The factor of one Cholesky QR pass, by one workgroup, from the G partial
@@ -194,21 +200,10 @@ __global__ __launch_bounds__(kThreads) void chol_factor_kernel(int w, float *ws,
     __shared__ float emax_w[4];
     const CholWork cw = carve<W>(ws);
     const int t = threadIdx.x;
-    if (G > kDirect) sum_partials<W>(cw.g, 1, w, Gs);
-    else sum_partials<W>(PASS == 2 ? cw.p2 : cw.p1, G, w, Gs);
-    __syncthreads();
+    const float e = G > kDirect ? load_gram<W>(cw.g, Gs) : sum_partials<W>(PASS == 2 ? cw.p2 : cw.p1, G, w, Gs);
+    const float emax = gram_dev_max(e, emax_w);
     bool first_order = false;
     if constexpr (PASS != 1) {
-        float e = 0.0f;
-        for (int q = t; q < W * W; q += kThreads) {
-            const int i = q % W, j = q / W;
-            if (i <= j) e = fmaxf(e, (float)fabs(Gs[i * LDG + j] - (i == j ? 1.0 : 0.0)));
-        }
-#pragma unroll
-        for (int mask = 32; mask > 0; mask >>= 1) e = fmaxf(e, __shfl_xor(e, mask, 64));
-        if ((t & 63) == 0) emax_w[t >> 6] = e;
-        __syncthreads();
-        const float emax = fmaxf(fmaxf(emax_w[0], emax_w[1]), fmaxf(emax_w[2], emax_w[3]));
         first_order = emax <= 1e-5f;  // NaN compares false: Cholesky path
         if (first_order) {
             for (int q = t; q < W * W; q += kThreads) {
@@ -264,7 +259,7 @@ __global__ __launch_bounds__(kThreads) void chol_apply_kernel(int m, int w, floa
     constexpr int CT = Shape<W>::CT, KS = Shape<W>::KS;
     constexpr int kAs = W * kApplyLd * 4;                       // the block, for the product
     constexpr int kQs = (PASS == 1) ? W * (kRows + 4) * 4 : 0;  // the stored Q1 rows, for their Gram
-    constexpr int kCb = (PASS == 1) ? 2 * Shape<W>::NT * 4 * 64 * 8 : 0;
+    constexpr int kCb = (PASS == 1) ? kGramLds<W> : 0;
     constexpr int kBytes = (kAs + kQs) > kCb ? (kAs + kQs) : kCb;
     __shared__ __attribute__((aligned(16))) char smem[kBytes];
     float *As = (float *)smem;
@@ -360,7 +355,7 @@ __global__ __launch_bounds__(kThreads) void chol_apply_kernel(int m, int w, floa
     }
     if constexpr (PASS == 1) {
         __syncthreads();
-        gram_finish<W>(g, (double *)smem, cw.p2 + (int64_t)blockIdx.x * Shape<W>::P);
+        gram_finish_shared<W>(g, (double *)smem, cw.p2 + (int64_t)blockIdx.x * Shape<W>::P);
     }
 }
 
@@ -398,46 +393,46 @@ __global__ __launch_bounds__(kThreads) void chol_apply_fused_kernel(int m, int w
     float av[kTT][KS];
     load_block_mfma<W>(A, lda, m, w, blockIdx.x * kRows, av);
 
-    if (G > kDirect) sum_partials<W>(cw.g, 1, w, Gs);  // reduced by chol_reduce_kernel
-    else sum_partials<W>(PASS == 2 ? cw.p2 : cw.p1, G, w, Gs);
-    __syncthreads();
-    bool first_order = false;
-    if constexpr (PASS != 1) {
-        // The panel (Q1, or a near-orthonormal input) has Gram I + E.  When
-        // max |E| <= 1e-5, R2 = I + U and R2^{-1} = I - U with
-        // U = triu(E, 1) + diag(E) / 2 agree with the Cholesky factor and its
-        // inverse to O(w |E|^2) <= 6.4e-9, far below the FP32 rounding of Q;
-        // otherwise (and for a zero column of Q1) the Cholesky runs.  Every
-        // workgroup sees the same E, so all take the same branch.
-        __shared__ float emax_w[4];
-        float e = 0.0f;
-        for (int q = t; q < W * W; q += kThreads) {
-            const int i = q % W, j = q / W;
-            if (i <= j) e = fmaxf(e, (float)fabs(Gs[i * LDG + j] - (i == j ? 1.0 : 0.0)));
-        }
+    __shared__ float emax_w[4];
+    const float e = G > kDirect ? load_gram<W>(cw.g, Gs) : sum_partials<W>(PASS == 2 ? cw.p2 : cw.p1, G, w, Gs);
+    const float emax = gram_dev_max(e, emax_w);
+    // A-operand slices of R^{-1}: rv[ct][s] = R^{-1}[4 s + l/16][16 ct + l%16]
+    // (zero for k > column, so column tile ct needs k-steps 0 .. 4 ct + 3).
+    double rv[CT][KS];
+    auto slices = [&](auto at) {
 #pragma unroll
-        for (int mask = 32; mask > 0; mask >>= 1) e = fmaxf(e, __shfl_xor(e, mask, 64));
-        if ((t & 63) == 0) emax_w[t >> 6] = e;
-        __syncthreads();
-        const float emax = fmaxf(fmaxf(emax_w[0], emax_w[1]), fmaxf(emax_w[2], emax_w[3]));
-        first_order = emax <= 1e-5f;  // NaN compares false: Cholesky path
-        if (first_order) {
-            for (int q = t; q < W * W; q += kThreads) {
-                const int i = q / W, j = q % W;
-                const double u = (i < j) ? Gs[i * LDG + j] : (i == j ? 0.5 * (Gs[i * LDG + i] - 1.0) : 0.0);
-                Rs[i * W + j] = (i == j ? 1.0 : 0.0) + u;
-                Ris[i * W + j] = (i == j ? 1.0 : 0.0) - u;
-            }
+        for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+            for (int s2 = 0; s2 < 4 * (ct + 1); ++s2) rv[ct][s2] = at(4 * s2 + (lane >> 4), 16 * ct + (lane & 15));
+    };
+    // The panel (Q1, or a near-orthonormal input) has Gram I + E.  When
+    // max |E| <= 1e-5, R2 = I + U and R2^{-1} = I - U with
+    // U = triu(E, 1) + diag(E) / 2 agree with the Cholesky factor and its
+    // inverse to O(w |E|^2) <= 6.4e-9, far below the FP32 rounding of Q;
+    // otherwise (and for a zero column of Q1) the Cholesky runs.  Every
+    // workgroup sees the same E, so all take the same branch (NaN compares
+    // false).  The inverse's slices then come straight from the Gram: the
+    // launch is a chain of latencies, and without R and R^{-1} passed through
+    // LDS, a second sweep for E and the unpacking of the reduced Gram it takes
+    // 13.3 us on average over a first and a second pass where it took 16.0
+    // (8192 x 64).
+    const bool first_order = PASS != 1 && emax <= 1e-5f;
+    auto upper = [&](int i, int j) { return i < j ? Gs[i * LDG + j] : (i == j ? 0.5 * (Gs[i * LDG + i] - 1.0) : 0.0); };
+    if (first_order) {
+        slices([&](int i, int j) { return (i == j ? 1.0 : 0.0) - upper(i, j); });
+        if constexpr (PASS == 2) {
+            for (int q = t; q < W * W; q += kThreads) Rs[q] = (q / W == q % W ? 1.0 : 0.0) + upper(q / W, q % W);
+            __syncthreads();
         }
-    }
-    if (!first_order) {
+    } else {
         const bool bad = factor<W>(Gs, Rs, Ris, d0);
         if (bad && t == 0 && blockIdx.x == 0 && status) atomicOr(status, 1);
+        __syncthreads();
+        slices([&](int i, int j) { return Ris[i * W + j]; });
     }
-    __syncthreads();
     if constexpr (PASS == 1) {
         if (blockIdx.x == 0)
-            for (int e = t; e < W * W; e += kThreads) cw.r1[e] = Rs[e];
+            for (int q = t; q < W * W; q += kThreads) cw.r1[q] = Rs[q];
     } else {
         // R (FP32, ldr): R1 itself (PASS 0) or R2 R1 (PASS 2, both upper,
         // FP64 then rounded once), four columns per round, column j by
@@ -446,6 +441,7 @@ __global__ __launch_bounds__(kThreads) void chol_apply_fused_kernel(int m, int w
         for (int j0 = blockIdx.x * 4; j0 < w; j0 += G * 4) {
             const int c = t >> 6, j = j0 + c, i = t & 63;
             if constexpr (PASS == 2) {
+                __syncthreads();  // every wave has its slices; the round before has been read
                 if (j < w && i < W) Gs[c * LDG + i] = (i <= j) ? cw.r1[i * W + j] : 0.0;
                 __syncthreads();
             }
@@ -456,22 +452,15 @@ __global__ __launch_bounds__(kThreads) void chol_apply_fused_kernel(int m, int w
                     // below-j entries are zeros, so the sum is the same.
 #pragma unroll
                     for (int k = 0; k < W; ++k) s = fma(Rs[i * W + k], Gs[c * LDG + k], s);
+                } else if (first_order) {
+                    s = (i == j ? 1.0 : 0.0) + upper(i, j);
                 } else {
                     s = Rs[i * W + j];
                 }
                 R[i + (int64_t)j * ldr] = (i <= j) ? (float)s : 0.0f;
             }
-            if constexpr (PASS == 2) __syncthreads();
         }
     }
-
-    // A-operand slices of R^{-1}: rv[ct][s] = R^{-1}[4 s + l/16][16 ct + l%16]
-    // (zero for k > column, so column tile ct needs k-steps 0 .. 4 ct + 3).
-    double rv[CT][KS];
-#pragma unroll
-    for (int ct = 0; ct < CT; ++ct)
-#pragma unroll
-        for (int s2 = 0; s2 < 4 * (ct + 1); ++s2) rv[ct][s2] = Ris[(4 * s2 + (lane >> 4)) * W + 16 * ct + (lane & 15)];
 
     Gram<W> g;
     gram_zero<W>(g);
@@ -510,7 +499,7 @@ __global__ __launch_bounds__(kThreads) void chol_apply_fused_kernel(int m, int w
     }
     if constexpr (PASS == 1) {
         __syncthreads();
-        gram_finish<W>(g, Cb, cw.p2 + (int64_t)blockIdx.x * Shape<W>::P);
+        gram_finish_shared<W>(g, Cb, cw.p2 + (int64_t)blockIdx.x * Shape<W>::P);
     }
 }
 
@@ -535,7 +524,7 @@ int launch_cholqr(hipStream_t s, int m, int w, float *A, int lda, float *R, int 
     hipLaunchKernelGGL(chol_gram_kernel<W>, dim3(G), dim3(kThreads), 0, s, m, w, (const float *)A, (int64_t)lda, work);
     ++n;
     if (G > kDirect) {
-        hipLaunchKernelGGL(chol_reduce_kernel<W>, rgrid, dim3(256), 0, s, cw.p1, G, cw.g);
+        hipLaunchKernelGGL(chol_reduce_kernel<W>, rgrid, dim3(256), 0, s, cw.p1, G, w, cw.g);
         ++n;
     }
     auto pass = [&](auto P) {
@@ -558,7 +547,7 @@ int launch_cholqr(hipStream_t s, int m, int w, float *A, int lda, float *R, int 
     }
     pass(std::integral_constant<int, 1>());
     if (G > kDirect) {
-        hipLaunchKernelGGL(chol_reduce_kernel<W>, rgrid, dim3(256), 0, s, cw.p2, G, cw.g);
+        hipLaunchKernelGGL(chol_reduce_kernel<W>, rgrid, dim3(256), 0, s, cw.p2, G, w, cw.g);
         ++n;
     }
     pass(std::integral_constant<int, 2>());
