@@ -39,6 +39,15 @@ int panel_tsqr(hipStream_t s, int m, int w, float *A, int lda, float *R, int ldr
 // one pass, two launches, for panels with condition number near 1); *status
 // gets bit 0 set on a numerically rank-deficient or non-finite Gram pivot.
 // The workspace depends on whether w is above 32.
+// up: the panel is A - Q C (Q m x k, k <= 64, outside the panel; C k x w),
+// formed in place in the same pass as its first Gram.
+struct PanelUpdate {
+    const float *Q;
+    int64_t ldq;
+    const float *C;
+    int64_t ldc;
+    int k;
+};
 int64_t panel_chol_work_floats(int w);
 int panel_cholqr2(hipStream_t s, int m, int w, float *A, int lda, float *R, int ldr, float *work, int64_t lwork,
-                  int *status, int *launches, bool once = false);
+                  int *status, int *launches, bool once = false, const PanelUpdate *up = nullptr);

@@ -101,15 +101,21 @@ template <int W> struct BlockRegs {
             }
         }
     }
+    // Either form; last: the last block inside (inside_last).
+    __device__ __forceinline__ void load_block(const float *A, int64_t lda, int m, int w, int b, int last)
+    {
+        if (b <= last) load_inside(A, lda, b * kRows);
+        else load(A, lda, m, w, b * kRows);
+    }
     // All W columns of 64 rows that all lie inside the panel, at any dword
     // alignment and without a branch (a branch around a load makes the
     // compiler wait at the join for every load in flight).
     __device__ __forceinline__ void load_inside(const float *A, int64_t lda, int r0)
     {
         const int t = threadIdx.x;
+        const float *src = A + (int64_t)(t >> 4) * lda + r0 + 4 * (t & 15);
 #pragma unroll
-        for (int j = 0; j < NV; ++j)
-            v[j] = *(const floatx4u *)(A + (int64_t)((t >> 4) + 16 * j) * lda + r0 + 4 * (t & 15));
+        for (int j = 0; j < NV; ++j) v[j] = *(const floatx4u *)(src + 16 * j * lda);  // (the same step for all lanes)
     }
     __device__ __forceinline__ void store_ld(float *Qs, int ld) const
     {
@@ -168,16 +174,133 @@ __global__ __launch_bounds__(kThreads) void chol_gram_kernel(int m, int w, const
             product();
         }
     } else {
-        if (b < nblk) r0.load(A, lda, m, w, b * kRows);
-        if (b + G < nblk) r1.load(A, lda, m, w, (b + G) * kRows);
+        if (b < nblk) r0.load_block(A, lda, m, w, b, last);
+        if (b + G < nblk) r1.load_block(A, lda, m, w, b + G, last);
     }
     for (int it = 0; b < nblk; b += G, ++it) {
         if (it & 1) block(r1); else block(r0);
         if (b + 2 * G < nblk) {
-            if (it & 1) r1.load(A, lda, m, w, (b + 2 * G) * kRows);
-            else r0.load(A, lda, m, w, (b + 2 * G) * kRows);
+            if (it & 1) r1.load_block(A, lda, m, w, b + 2 * G, last);
+            else r0.load_block(A, lda, m, w, b + 2 * G, last);
         }
         product();
+    }
+    __syncthreads();
+    gram_finish_shared<W>(g, (double *)smem, cw.p1 + (int64_t)blockIdx.x * Shape<W>::P);
+}
+
+// A -= Q C (Q: m x k, k <= 64; C: k x w) and the partial Gram of the result,
+// in one pass over both: the update of a node whose second half is a leaf, and
+// that leaf's first launch.  The Gram kernel's blocks and grid, so the partials
+// are the same; the product is a chain of FP32 MFMA steps over k and one fused
+// multiply-add with A, as in the separate update, so A keeps its bits too.
+// Each wave forms the 16 rows whose Gram it takes, so between the two products
+// the rows go through LDS without a barrier.  Q's and A's rows come in 256-byte
+// runs a block ahead (4600 cycles of MFMA a block and wave, two waves a SIMD); C stays in LDS in operand order (lane l of step
+// 4 s + u: column l % 16, k = 16 s + 4 u + l / 16).
+// Bound by memory when tall.  1048576 x 64 with k = 64: 233 us, against 188 for
+// the update and 104 for the Gram; 262144 rows 59 against 45 and 29; 8192 rows
+// 9.7 against 5.1 and 5.8, with a launch less.
+template <int W>
+__global__ __launch_bounds__(kThreads, 2) void chol_update_gram_kernel(int m, int w, float *A, int64_t lda, float *ws, int k,
+                                                                    const float *Q, int64_t ldq, const float *C,
+                                                                    int64_t ldc)
+{
+    constexpr int KM = 64, LDC = KM + 4, CT = Shape<W>::CT;
+    constexpr int kAs = KM * (kRows + 16) * 4, kQs = W * (kRows + 4) * 4, kCs = W * LDC * 4, kCb = kGramLds<W>;
+    constexpr int kBytes = (kAs + kQs + kCs) > kCb ? (kAs + kQs + kCs) : kCb;
+    __shared__ __attribute__((aligned(16))) char smem[kBytes];
+    float *As = (float *)smem, *Qs = (float *)(smem + kAs), *Cs = (float *)(smem + kAs + kQs);
+    const CholWork cw = carve<W>(ws);
+    const int nblk = (m + kRows - 1) / kRows;
+    const int G = gridDim.x;
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, li = lane & 15, lk = lane >> 4;
+    const int lrow = wv * 16 + li;  // row within the block
+    Gram<W> g;
+    gram_zero<W>(g);
+    struct Rows {
+        BlockRegs<KM> q;
+        BlockRegs<W> a;
+    } r;
+    int b = blockIdx.x;
+    const int last = k == KM ? inside_last(m, w, W) : -1;
+    auto load = [&](Rows &r, int b) {
+        r.q.load_block(Q, ldq, m, k, b, last);
+        r.a.load_block(A, lda, m, w, b, last);
+    };
+    auto block = [&]() {
+        __syncthreads();  // the previous block has been read
+        r.q.store_ld(As, kRows + 16);
+        r.a.store(Qs);
+        __syncthreads();
+    };
+    auto product = [&](auto inside) {
+        const int row = b * kRows + lrow;
+        floatx4 acc[CT];
+#pragma unroll
+        for (int c = 0; c < CT; ++c) acc[c] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int s = 0; s < KM / 16; ++s) {
+            float q[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) q[u] = As[(16 * s + 4 * u + lk) * (kRows + 16) + lrow];
+            floatx4 a[CT];
+#pragma unroll
+            for (int c = 0; c < CT; ++c) a[c] = *(const floatx4 *)&Cs[(16 * c + li) * LDC + 16 * s + 4 * lk];
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+#pragma unroll
+                for (int c = 0; c < CT; ++c) acc[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[c][u], q[u], acc[c], 0, 0, 0);
+        }
+        // acc[c][e]: row l % 16 of the wave's, column 16 c + 4 (l / 16) + e
+        float *out = A + row + 4 * lk * lda;
+#pragma unroll
+        for (int c = 0; c < CT; ++c)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int col = 16 * c + 4 * lk + e;
+                const bool ok = decltype(inside)::value || (row < m && col < w);
+                float *x = &Qs[col * (kRows + 4) + lrow];
+                const float v = ok ? fmaf(-1.0f, acc[c][e], *x) : 0.0f;
+                if (ok) out[(16 * c + e) * lda] = v;
+                *x = v;
+            }
+        __builtin_amdgcn_wave_barrier();  // the wave's own rows: its LDS accesses stay in order
+        gram_lds<W>(g, Qs, wv * 16);
+    };
+    static_assert(kTT == 1, "a wave updates the 16 rows whose Gram it forms");
+    load(r, b);
+    {
+        constexpr int N = W * KM / kThreads, S = kThreads / KM;
+        const int kk = threadIdx.x % KM, c0 = threadIdx.x / KM;
+        float x[N];
+#pragma unroll
+        for (int n = 0; n < N; ++n) x[n] = C[min(kk, k - 1) + (int64_t)min(c0 + S * n, w - 1) * ldc];
+#pragma unroll
+        for (int n = 0; n < N; ++n)
+            Cs[(c0 + S * n) * LDC + (kk & ~15) + 4 * (kk & 3) + ((kk >> 2) & 3)] =
+                (kk < k && c0 + S * n < w) ? x[n] : 0.0f;
+    }
+    auto step = [&]() {
+        block();
+        r.q.load_inside(Q, ldq, (b + G) * kRows);
+        r.a.load_inside(A, lda, (b + G) * kRows);
+        product(std::true_type());
+        b += G;
+    };
+    if (b <= last) {  // apart, as in the apply kernel; all there is below 512 blocks
+        block();
+        if (b + G < nblk) load(r, b + G);
+        product(std::true_type());
+        b += G;
+    }
+#pragma unroll 1
+    while (b + G <= last) step();
+#pragma unroll 1
+    for (; b < nblk; b += G) {
+        block();
+        if (b + G < nblk) load(r, b + G);
+        product(std::false_type());
     }
     __syncthreads();
     gram_finish_shared<W>(g, (double *)smem, cw.p1 + (int64_t)blockIdx.x * Shape<W>::P);
@@ -303,6 +426,7 @@ __global__ __launch_bounds__(kThreads) void chol_apply_kernel(int m, int w, floa
             for (int ct = 0; ct < CT; ++ct)
                 if (s2 < 4 * (ct + 1)) d[ct] = __builtin_amdgcn_mfma_f64_16x16x4f64(rv[ct][s2], (double)av[s2], d[ct], 0, 0, 0);
         // d[ct][r] = Q[row][16 ct + l/16 + 4 r]
+        float *out = A + row + (lane >> 4) * lda;
 #pragma unroll
         for (int ct = 0; ct < CT; ++ct)
 #pragma unroll
@@ -310,7 +434,7 @@ __global__ __launch_bounds__(kThreads) void chol_apply_kernel(int m, int w, floa
                 const int col = 16 * ct + (lane >> 4) + 4 * q;
                 const bool ok = decltype(inside)::value || (row < m && col < w);
                 const float v = ok ? (float)d[ct][q] : 0.0f;
-                if (ok) A[row + (int64_t)col * lda] = v;
+                if (ok) out[(16 * ct + 4 * q) * lda] = v;
                 if constexpr (PASS == 1) Qs[col * (kRows + 4) + lrow] = v;
             }
         if constexpr (PASS == 1) {
@@ -341,15 +465,15 @@ __global__ __launch_bounds__(kThreads) void chol_apply_kernel(int m, int w, floa
 #pragma unroll 1
         while (b + 3 * G <= last) pair();
     } else {
-        if (b < nblk) r0.load(A, lda, m, w, b * kRows);
-        if (b + G < nblk) r1.load(A, lda, m, w, (b + G) * kRows);
+        if (b < nblk) r0.load_block(A, lda, m, w, b, last);
+        if (b + G < nblk) r1.load_block(A, lda, m, w, b + G, last);
     }
 #pragma unroll 1
     for (int it = 0; b < nblk; b += G, ++it) {
         if (it & 1) block(r1); else block(r0);
         if (b + 2 * G < nblk) {
-            if (it & 1) r1.load(A, lda, m, w, (b + 2 * G) * kRows);
-            else r0.load(A, lda, m, w, (b + 2 * G) * kRows);
+            if (it & 1) r1.load_block(A, lda, m, w, b + 2 * G, last);
+            else r0.load_block(A, lda, m, w, b + 2 * G, last);
         }
         product(b, std::false_type());
     }
@@ -510,7 +634,7 @@ constexpr int kFusedBlocks = 256;
 
 template <int W>
 int launch_cholqr(hipStream_t s, int m, int w, float *A, int lda, float *R, int ldr, float *work, int *status,
-                  int G, bool once)
+                  int G, bool once, const PanelUpdate *up)
 {
     const CholWork cw = carve<W>(work);
     const int nblk = (m + kRows - 1) / kRows;
@@ -521,7 +645,11 @@ int launch_cholqr(hipStream_t s, int m, int w, float *A, int lda, float *R, int 
     const bool fused = nblk <= kFusedBlocks;
     const dim3 rgrid((Shape<W>::P + 31) / 32);
     int n = 0;
-    hipLaunchKernelGGL(chol_gram_kernel<W>, dim3(G), dim3(kThreads), 0, s, m, w, (const float *)A, (int64_t)lda, work);
+    if (up)
+        hipLaunchKernelGGL(chol_update_gram_kernel<W>, dim3(G), dim3(kThreads), 0, s, m, w, A, (int64_t)lda, work, up->k,
+                           up->Q, up->ldq, up->C, up->ldc);
+    else
+        hipLaunchKernelGGL(chol_gram_kernel<W>, dim3(G), dim3(kThreads), 0, s, m, w, (const float *)A, (int64_t)lda, work);
     ++n;
     if (G > kDirect) {
         hipLaunchKernelGGL(chol_reduce_kernel<W>, rgrid, dim3(256), 0, s, cw.p1, G, w, cw.g);
@@ -559,14 +687,15 @@ int launch_cholqr(hipStream_t s, int m, int w, float *A, int lda, float *R, int 
 int64_t panel_chol_work_floats(int w) { return w <= 32 ? work_floats<32>() : work_floats<64>(); }
 
 int panel_cholqr2(hipStream_t s, int m, int w, float *A, int lda, float *R, int ldr, float *work, int64_t lwork,
-                  int *status, int *launches, bool once)
+                  int *status, int *launches, bool once, const PanelUpdate *up)
 {
+    if (up && (up->k < 1 || up->k > kWMax)) return LATER_ERR_SHAPE;
     if (w < 1 || w > kWMax || m < w) return LATER_ERR_SHAPE;
     if (lwork < panel_chol_work_floats(w)) return LATER_ERR_WORKSPACE;
     const int nblk = (m + kRows - 1) / kRows;
     const int G = nblk < kMaxGroups ? nblk : kMaxGroups;
-    const int n = (w <= 32) ? launch_cholqr<32>(s, m, w, A, lda, R, ldr, work, status, G, once)
-                            : launch_cholqr<64>(s, m, w, A, lda, R, ldr, work, status, G, once);
+    const int n = (w <= 32) ? launch_cholqr<32>(s, m, w, A, lda, R, ldr, work, status, G, once, up)
+                            : launch_cholqr<64>(s, m, w, A, lda, R, ldr, work, status, G, once, up);
     HIP_OK(hipGetLastError());
     if (launches) *launches += n;
     return LATER_OK;

@@ -343,8 +343,15 @@ int qr_rec(Run &r, int m, int n, float *A, int64_t lda, float *R, int64_t ldr, i
     rc = gemm_proj(r.s, p, m, n1, n2, A, lda, A2, lda, R12, ldr, chunk, bexp, aexp, r.gemm, r.gemm_n,
                    &r.launches, pre_proj ? &q1h : nullptr, pre_proj ? &a2h : nullptr);
     if (rc) return rc;
-    // A2 -= Q1 R12    (QR/later_rgsqrf.cu:51-56); R12's column exponents
-    // replace A2's.
+    // A2 -= Q1 R12    (QR/later_rgsqrf.cu:51-56), in one pass with A2's first
+    // Gram where A2 is a Cholesky leaf of its own.
+    if (chol_panel(r.o.panel) && n1 <= 64 && n2 <= 64 && pu == LATER_GEMM_F32 && !f64 && !r.node_reorth) {
+        const PanelUpdate up = {A, lda, R12, ldr, n1};
+        if (depth + 1 > r.depth) r.depth = depth + 1;
+        return panel_cholqr2(r.s, m, n2, A2, (int)lda, R + n1 + (int64_t)n1 * ldr, (int)ldr, r.panel, r.panel_n, r.status,
+                             &r.launches, r.chol_once || r.o.panel == LATER_PANEL_CHOLQR1, &up);
+    }
+    // Otherwise R12's column exponents replace A2's.
     if (pre) {
         if ((rc = ensure_q<true>(r, pu, m, c0, n1, A, lda, aexp_u))) return rc;
         if (scaled(pu))

@@ -173,3 +173,25 @@ def test_streamed_products(later, oracle, m, n1, n2, pad, prec, extra):
     assert np.all(np.abs(P - Q.T @ B) <= (m + 2 + extra) * u * (np.abs(Q).T @ np.abs(B)) + m * 2.0 ** -22 * (extra > 16))
     assert np.all(np.abs(U - (B - Q @ C)) <= (n1 + 2 + extra) * u * (np.abs(Q) @ np.abs(C)) + 2 * u * np.abs(B)
                   + n1 * 2.0 ** -22 * (extra > 16))
+
+
+# A node whose second half is a Cholesky leaf: update and first Gram in one
+# pass.  Against the same steps one by one (leaf, projection, update, leaf), for
+# both kernel widths, fewer and more blocks than workgroups, ragged rows and any
+# leading dimension: the same bits.
+@pytest.mark.parametrize("m", [128, 161, 4099, 33000, 131072 + 70, 300003])
+@pytest.mark.parametrize("n,pad", [(65, 1), (96, 0), (97, 3), (127, 2), (128, 0), (128, 1)])
+@pytest.mark.parametrize("panel", ["PANEL_CHOLQR1", "PANEL_CHOLQR2"])
+def test_update_with_leaf_gram(later, oracle, m, n, pad, panel):
+    o = later.opts("mixed", reorth=0, panel=getattr(later, panel))
+    A = _dev(later, oracle.gen_uniform(m, n, 11, 6), pad)
+    X, R = _dev(later, _np(A), pad), later.colmajor(n, n, ld=n + pad)
+    later.rgsqrf(A, o=o, R=R)
+    S = later.colmajor(n, n, ld=n + pad)
+    X1, X2 = X[:, :64], X[:, 64:]
+    later.rgsqrf(X1, R=S[:64, :64], o=o)
+    later.gemm_proj(X1, X2, S[:64, 64:], later.GEMM_F32)
+    later.gemm_update(X1, S[:64, 64:], X2, later.GEMM_F32)
+    later.rgsqrf(X2, R=S[64:, 64:], o=o)
+    assert np.array_equal(_np(A), _np(X))
+    assert np.array_equal(np.triu(_np(R)), np.triu(_np(S)))
