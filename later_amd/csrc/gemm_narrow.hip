@@ -199,34 +199,37 @@ __global__ __launch_bounds__(kThreads, 2) void update_narrow_kernel(int M, int N
 } // namespace
 
 // Measured against the general kernel's 64 x 64 tiles (us, 16384 rows unless
-// said): 32 x 32 9.0 against 19.6, 64 x 64 9.6 / 17.8, 128 x 128 16.3 / 19.5,
-// with the reduction of the partials.  A 32 x 32 tile reads its rows more often
-// than a 64 x 64 one where both sides are wide; that is paid back while the
-// launch is latency-bound: 64 x 64 at 131072 rows 43.9 / 47.8, at 262144 63.4 /
-// 58.4; 128 x 128 at 32768 25.0 / 27.7, at 65536 44.9 / 44.9.  Up to 1.5 times
-// the traffic it stays ahead at every height (96 x 64 at 524288: 131 / 146).
+// said): 32 x 32 8.9 against 13.5, 64 x 64 9.5 / 13.6, 32 x 128 9.3 / 13.8, with
+// the reduction of the partials.  Where both sides are wide, a 32 x 32 tile
+// reads its rows more often than a 64 x 64 one; that is paid back while the
+// launch is latency-bound: 64 x 64 at 32768 rows 13.9 / 16.2, at 65536 22.6 /
+// 21.4; 128 x 128 at 8192 10.6 / 12.9, at 16384 15.9 / 15.3; 96 x 64 at 16384
+// 14.0 / 15.5, at 32768 21.4 / 18.2.  At equal traffic it is ahead at every
+// height (32 x 128 at 524288: 91 / 103, 64 x 32 at 1048576 114 / 119).
 bool gemm_proj_narrow(hipStream_t s, int m, int n1, int n2, const float *Q, int64_t ldq, const float *B, int64_t ldb,
                       float *C, int64_t ldc, int nsplit, int kper, float *partial)
 {
     if (n1 > 128 || n2 > 128) return false;
     const int64_t tiles = ceil_div64(n1, 32) * ceil_div64(n2, 32);
     const int64_t reads = 64 * tiles, reads64 = 128 * ceil_div64(n1, 64) * ceil_div64(n2, 64);  // columns read per row
-    if (2 * reads > 3 * reads64 && tiles * m > (1 << 19)) return false;
+    if (reads > reads64 && tiles * m > (1 << 17)) return false;
     hipLaunchKernelGGL(proj_narrow_kernel, dim3((unsigned)nsplit, (unsigned)tiles), dim3(kThreads), 0, s, n1, n2, m, kper,
                        Q, ldq, B, ldb, C, ldc, partial);
     return true;
 }
 
-// Against the general kernel (us): depth 32 ahead at every height (32 columns:
-// 16384 rows 4.2 / 7.7, 1048576 91 / 137); depth 64, 64 columns: 16384 rows
-// 5.6 / 8.8, 524288 84 / 95, 1048576 286 / 225 (past the 256 MB cache its
-// 64-byte row segments lose to whole 256-byte tiles); depth 128, 128 columns:
-// 4096 rows 6.0 / 10.1, 16384 13.4 / 14.0, 65536 46.4 / 43.3.
+// Against the general kernel (us): depth 32 ahead or level while the operands
+// fit the 256 MB cache (32 columns: 16384 rows 4.2 / 4.8, 262144 23.6 / 26.3; 128
+// columns: 262144 rows 54 / 57, 524288 202 / 149: past it, its 64-byte row
+// segments lose to whole 256-byte tiles); depth 64 up to two workgroups a CU (64
+// columns: 8192 rows 4.4 / 5.4, 16384 5.7 / 5.9, 32768 8.8 / 8.2); deeper, up to
+// one (128 columns: 4096 rows 6.0 / 7.2, 8192 7.9 / 7.6, 16384 13.1 / 11.1).
 bool gemm_update_narrow(hipStream_t s, int M, int N, int K, float alpha, const float *Q, int64_t ldq, const float *C,
                         int64_t ldc, float *B, int64_t ldb, bool f64)
 {
     const int64_t cols = ceil_div64(N, 64), blocks = ceil_div64(M, 32);
-    if (K > 128 || cols > 65535 || (K > 64 && M > 16384) || (K > 32 && (int64_t)M * N > (1 << 25))) return false;
+    if (K > 128 || cols > 65535) return false;
+    if (K <= 32 ? (int64_t)M * N > (1 << 25) : blocks * cols > (K <= 64 ? 512 : 256)) return false;
     const dim3 grid((unsigned)(blocks < 2048 ? blocks : 2048), (unsigned)cols);
     const int d = f64 ? 1 : 0;
     if (K <= 32)
