@@ -195,3 +195,18 @@ def test_update_with_leaf_gram(later, oracle, m, n, pad, panel):
     later.rgsqrf(X2, R=S[64:, 64:], o=o)
     assert np.array_equal(_np(A), _np(X))
     assert np.array_equal(np.triu(_np(R)), np.triu(_np(S)))
+
+
+# Projections of many splits (97 and more): their reduction's rounds, ragged
+# elements of its last workgroup, FP32 and FP64 partials.  Bounds as above (a
+# split's FP32 chain is shorter than m; FP64 folds keep chains to 256).
+@pytest.mark.parametrize("m", [24900, 40001, 131072 + 5])
+@pytest.mark.parametrize("n1,n2", [(64, 64), (33, 17), (1, 3), (128, 100)])
+@pytest.mark.parametrize("prec,chunk", [("GEMM_F32", 0), ("GEMM_F16X6", 256)])
+def test_many_splits(later, oracle, m, n1, n2, prec, chunk):
+    A, B = oracle.gen_uniform(m, n1, 1, 1), oracle.gen_uniform(m, n2, 2, 2)
+    C = _np(later.gemm_proj(_dev(later, A, 1), _dev(later, B), later.colmajor(n1, n2, ld=n1 + 1),
+                            getattr(later, prec), chunk))
+    A, B = A.astype(np.float64), B.astype(np.float64)
+    k = chunk + 16 if chunk else 2048
+    assert np.all(np.abs(C - A.T @ B) <= (k + 2) * 2.0 ** -24 * (np.abs(A).T @ np.abs(B)))
