@@ -1336,28 +1336,38 @@ __global__ __launch_bounds__(256) void splitk_reduce_lds_kernel(int M, int N, in
 }
 
 // Per-column exponents e_j with max_i |X_ij| 2^e_j in [2^14, 2^15) (0 for a
-// zero column).  One 256-thread workgroup per column, 16-byte loads where the
-// column is aligned (the maximum does not depend on the order).
-// Exponent of column x (m values) by the whole 256-thread workgroup:
+// zero column).  One workgroup per column, 16-byte loads where the column is
+// aligned (the maximum does not depend on the order).
+// Exponent of column x (m values) by the whole workgroup of T threads:
 // e with max |x| 2^e in [2^14, 2^15) (0 for a zero or non-finite maximum).
-__device__ __forceinline__ int column_exp(int m, const float *x)
+template <int T> __device__ __forceinline__ int column_exp(int m, const float *x)
 {
-    __shared__ float wmax[4];
+    __shared__ float wmax[T / 64];
     float mx = 0.0f;
     const int head = (int)min((int64_t)m, (int64_t)((16 - ((uintptr_t)x & 15)) & 15) / 4);
-    for (int i = threadIdx.x; i < head; i += 256) mx = fmaxf(mx, fabsf(x[i]));
+    for (int i = threadIdx.x; i < head; i += T) mx = fmaxf(mx, fabsf(x[i]));
     const int nv = (m - head) / 4;
     const floatx4 *xv = (const floatx4 *)(x + head);
-    for (int v = threadIdx.x; v < nv; v += 256) {
-        const floatx4 q = xv[v];
+    auto take = [&](floatx4 q) {
         mx = fmaxf(mx, fmaxf(fmaxf(fabsf(q[0]), fabsf(q[1])), fmaxf(fabsf(q[2]), fabsf(q[3]))));
+    };
+    constexpr int U = 8;  // loads in flight per thread
+    int v = threadIdx.x;
+    for (; v + (U - 1) * T < nv; v += U * T) {
+        floatx4 q[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) q[u] = xv[v + u * T];
+#pragma unroll
+        for (int u = 0; u < U; ++u) take(q[u]);
     }
-    for (int i = head + 4 * nv + threadIdx.x; i < m; i += 256) mx = fmaxf(mx, fabsf(x[i]));
+    for (; v < nv; v += T) take(xv[v]);
+    for (int i = head + 4 * nv + threadIdx.x; i < m; i += T) mx = fmaxf(mx, fabsf(x[i]));
 #pragma unroll
     for (int mask = 32; mask > 0; mask >>= 1) mx = fmaxf(mx, __shfl_xor(mx, mask, 64));
     if ((threadIdx.x & 63) == 0) wmax[threadIdx.x >> 6] = mx;
     __syncthreads();
-    mx = fmaxf(fmaxf(wmax[0], wmax[1]), fmaxf(wmax[2], wmax[3]));
+#pragma unroll
+    for (int w = 0; w < T / 64; ++w) mx = fmaxf(mx, wmax[w]);
     int ex = 0;
     if (mx > 0.0f && mx < INFINITY) {
         int fe;
@@ -1367,10 +1377,14 @@ __device__ __forceinline__ int column_exp(int m, const float *x)
     return ex;
 }
 
-__global__ __launch_bounds__(256) void colexp_kernel(int m, int n, const float *X, int64_t ldx, int *e)
+// Bound by the loads that one column's workgroup keeps in flight: T = 1024 for
+// columns of more than kColexpRows values (128 columns of 262144: 115 us with 256
+// threads and a load each, 28 with 1024 and eight).
+constexpr int kColexpRows = 16384;
+template <int T> __global__ __launch_bounds__(T) void colexp_kernel(int m, int n, const float *X, int64_t ldx, int *e)
 {
     const int j = blockIdx.x;
-    const int ex = column_exp(m, X + (int64_t)j * ldx);
+    const int ex = column_exp<T>(m, X + (int64_t)j * ldx);
     if (threadIdx.x == 0) e[j] = ex;
 }
 
@@ -1520,7 +1534,7 @@ __global__ __launch_bounds__(256) void split_exp_kernel(int rows, const float *X
         }
         return;
     }
-    const int ex = column_exp(rows, x);
+    const int ex = column_exp<256>(rows, x);
     if (threadIdx.x == 0) col_exp[j] = ex;
     const float sc = ldexpf(1.0f, ex);
     const int prow = (rows + 63) / 64 * 64;
@@ -1914,7 +1928,8 @@ int gemm_nn(hipStream_t s, int prec, int M, int N, int K, float alpha, const flo
 int gemm_colexp(hipStream_t s, int m, int n, const float *X, int64_t ldx, int *e, int *launches)
 {
     if (n <= 0) return LATER_OK;
-    hipLaunchKernelGGL(colexp_kernel, dim3(n), dim3(256), 0, s, m, n, X, ldx, e);
+    if (m > kColexpRows) hipLaunchKernelGGL(colexp_kernel<1024>, dim3(n), dim3(1024), 0, s, m, n, X, ldx, e);
+    else hipLaunchKernelGGL(colexp_kernel<256>, dim3(n), dim3(256), 0, s, m, n, X, ldx, e);
     HIP_OK(hipGetLastError());
     if (launches) ++*launches;
     return LATER_OK;

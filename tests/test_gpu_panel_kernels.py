@@ -210,3 +210,19 @@ def test_many_splits(later, oracle, m, n1, n2, prec, chunk):
     A, B = A.astype(np.float64), B.astype(np.float64)
     k = chunk + 16 if chunk else 2048
     assert np.all(np.abs(C - A.T @ B) <= (k + 2) * 2.0 ** -24 * (np.abs(A).T @ np.abs(B)))
+
+
+# Column exponents on both sides of the tall kernel's line, with the largest
+# entry in the first row, the last row or the last whole vector, columns far from
+# 1 and any address: a wrong exponent overflows FP16 or loses the column.  Bound
+# as above (FP64 folds every 256 rows).
+@pytest.mark.parametrize("m", [16384, 16385, 32768 + 5, 70001])
+@pytest.mark.parametrize("pad", [0, 1, 2])
+def test_tall_column_exponents(later, oracle, m, pad):
+    A, B = oracle.gen_uniform(m, 40, 1, 1), oracle.gen_uniform(m, 6, 2, 2)
+    for j, (i, p) in enumerate([(0, 40), (m - 1, -40), (m - 6, 20), (m // 2, -20), (1, 0), (m - 2, 3)]):
+        B[i, j] = 1000.0
+        B[:, j] = np.ldexp(B[:, j], p)
+    C = _np(later.gemm_proj(_dev(later, A, pad), _dev(later, B, pad), later.colmajor(40, 6), later.GEMM_F16X6, 256))
+    A, B = A.astype(np.float64), B.astype(np.float64)
+    assert np.all(np.abs(C - A.T @ B) <= (256 + 18) * 2.0 ** -24 * (np.abs(A).T @ np.abs(B)))
