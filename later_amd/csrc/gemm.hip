@@ -1872,7 +1872,7 @@ int gemm_proj(hipStream_t s, int prec, int m, int n1, int n2, const float *Q, in
     if (ns > 1) {
         const int64_t tot = (int64_t)n1 * n2;
         dim3 grid((unsigned)ceil_div64(tot, 256)), lgrid((unsigned)ceil_div64(tot, ch64 ? 16 : 32));
-        const bool many = ns > 96;  // 80 splits 4.6 us against 4.0 to 4.8, 128 5.7 / 4.1, 256 9.8 / 5.3
+        const bool many = ns > 96;  // 80 splits level (4.4 to 4.8 us), 128 5.7 against 4.1, 256 9.8 against 5.3
         if (many && ch64)
             hipLaunchKernelGGL(splitk_reduce_lds_kernel<true>, lgrid, dim3(256), 0, s, n1, n2, ns, work, C, ldc);
         else if (many)

@@ -10,8 +10,8 @@
 //           triangle as a partial (a fixed-tree reduction kernel adds them
 //           when there are more than 32);
 //   factor  one workgroup adds the partials in a fixed order, factors
-//           G = R^T R and inverts R (FP64, one wave per 32 x 32 diagonal
-//           block, columns in registers), and stores R^{-1} (and R);
+//           G = R^T R and inverts R (FP64, in 16-column blocks), and stores
+//           R^{-1} (and R);
 //   apply   up to 1024 workgroups form q = a R^{-1} for their rows on FP64
 //           MFMA and store Q in FP32; in the first of two passes they also
 //           form the partial Grams of the stored Q1 for the second, which
