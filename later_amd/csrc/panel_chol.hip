@@ -12,7 +12,7 @@
 //   factor  one workgroup adds the partials in a fixed order, factors
 //           G = R^T R and inverts R (FP64, in 16-column blocks), and stores
 //           R^{-1} (and R);
-//   apply   up to 1024 workgroups form q = a R^{-1} for their rows on FP64
+//   apply   the same grid forms q = a R^{-1} for its rows on FP64
 //           MFMA and store Q in FP32; in the first of two passes they also
 //           form the partial Grams of the stored Q1 for the second, which
 //           repeats the factor and apply on Q1 and sets R = R2 R1.
@@ -371,9 +371,10 @@ __global__ __launch_bounds__(kThreads) void chol_factor_kernel(int w, float *ws,
 // four column tiles' accumulation chains are interleaved k-step by k-step
 // (up to four independent MFMAs in flight); D's lanes walk 16 consecutive
 // rows of one column (64-byte stores).  PASS 1 also forms the partial Gram
-// of the stored Q1 rows into p2[blockIdx.x] (then the grid is the Gram
-// kernel's).  Bound by memory (110 us for 1048576 x 64 at a copy's rate);
-// without a branch around a load or a store it takes 127 us, 152 before.
+// of the stored Q1 rows into p2[blockIdx.x].  The grid is the Gram kernel's, two
+// workgroups a CU, which is what the registers hold: 1048576 x 64 takes 120 us,
+// 127 in two rounds on 1024 workgroups (262144 rows 35 and 39).  Bound by memory
+// (110 us at a copy's rate); 152 us with branches around the loads and stores.
 constexpr int kApplyLd = kRows + 16;
 
 template <int PASS, int W>
@@ -627,9 +628,6 @@ __global__ __launch_bounds__(kThreads) void chol_apply_fused_kernel(int m, int w
     }
 }
 
-// Workgroups of the apply kernels without a partial Gram: several per CU, so
-// tall panels keep enough loads in flight.
-constexpr int kMaxApplyGroups = 1024;
 constexpr int kFusedBlocks = 256;
 
 template <int W>
@@ -638,7 +636,6 @@ int launch_cholqr(hipStream_t s, int m, int w, float *A, int lda, float *R, int 
 {
     const CholWork cw = carve<W>(work);
     const int nblk = (m + kRows - 1) / kRows;
-    const int Ga = nblk < kMaxApplyGroups ? nblk : kMaxApplyGroups;
     // Up to kFusedBlocks blocks every apply workgroup forms the factor itself
     // (the latency of a separate factor launch outweighs the redundancy);
     // taller panels factor once and apply with more workgroups.
@@ -664,7 +661,7 @@ int launch_cholqr(hipStream_t s, int m, int w, float *A, int lda, float *R, int 
         } else {
             hipLaunchKernelGGL((chol_factor_kernel<PASS, W>), dim3(1), dim3(kThreads), 0, s, w, work, G, R,
                                (int64_t)ldr, status);
-            hipLaunchKernelGGL((chol_apply_kernel<PASS, W>), dim3(PASS == 1 ? G : Ga), dim3(kThreads), 0, s, m, w, A,
+            hipLaunchKernelGGL((chol_apply_kernel<PASS, W>), dim3(G), dim3(kThreads), 0, s, m, w, A,
                                (int64_t)lda, work);
             n += 2;
         }
