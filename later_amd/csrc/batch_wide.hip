@@ -14,8 +14,8 @@
 // of FP32 data one Cholesky QR leaves kappa^2 2^-53, far below the rounding of
 // Q's entries to FP32, and what is left of Q in P grows by kappa at most.  When
 // ||R||_F ||R^{-1}||_F (>= kappa, >= w) exceeds 4 w, or a pivot was bad, the
-// normalised panel is projected out of Q once more and factored again, so that
-// neither depends on the panel's condition.
+// normalised panel is projected out of Q once more (with reorthogonalisation)
+// and factored again, so that neither depends on the panel's condition.
 //
 // A chunk of 32 rows of [Q P] is staged in LDS column by column (stride 36:
 // 16-byte reads of 16 columns and 4-byte reads of 16 rows of every fourth
@@ -426,15 +426,16 @@ __device__ __forceinline__ void wide_factor(const WgTask &tk, char *lds, bool re
         p.lda = tk.lda;
         float *P = tk.A + (int64_t)c0 * tk.lda;
         // Step 0: S = Q^T P; 1 (reorth): P -= Q S, S = Q^T P again; 2: P -= Q S
-        // (c0 > 0) and G, factor, apply.  A panel that needs it goes on: 3:
-        // S = Q^T P of the normalised panel; 4 as 2.
+        // (c0 > 0) and G, factor, apply.  A panel that needs it goes on: 3
+        // (reorth, c0 > 0): S = Q^T P of the normalised panel; 4: as 2 with that
+        // S, and G alone without one (R^{-1} then lies in S's place).
         int step = c0 > 0 ? 0 : 2;
         for (;;) {
             const bool project = step < 2 || step == 3;
             if (step == 1) sweep<true, true>(p, P, lds);
             else if (project) sweep<false, true>(p, P, lds);
-            else if (c0 > 0) sweep<true, false>(p, P, lds);
-            else sweep<false, false>(p, P, lds);
+            else if (c0 > 0 && (step == 2 || reorth)) sweep<true, false>(p, P, lds);
+            else sweep<false, false>(p, P, lds);  // no S: the first panel, or step 4 without step 3
             if (project) {
                 // R's rows above the panel: S, + S, + S R1.
                 for (int e = threadIdx.x; e < c0 * p.w; e += kT) {

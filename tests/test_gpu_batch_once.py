@@ -1,0 +1,62 @@
+"""The batched QR's FP32 kernels with one projection (reorth = 0), where a panel
+behind the first may have to be factored a second time (GPU)."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+WIDE = 4
+
+
+def _run(later, mats, variant, form="fp32", reorth=0, pad=0):
+    As, Rs = [], []
+    for A in mats:
+        X = later.colmajor(A.shape[0], A.shape[1], ld=A.shape[0] + pad)
+        X.copy_(torch.from_numpy(np.ascontiguousarray(A)))
+        As.append(X)
+        Rs.append(later.colmajor(A.shape[1], A.shape[1], ld=A.shape[1] + pad))
+    tuning = None if variant is None else [variant] * later.BATCH_BUCKETS
+    plan = later.BatchWg(As, Rs, later.opts(form, reorth=reorth), tuning=tuning)
+    plan.execute()
+    torch.cuda.synchronize()
+    status = plan.status.cpu().numpy().copy()
+    plan.close()
+    return [(q.cpu().numpy().copy(order="F"), r.cpu().numpy().copy(order="F")) for q, r in zip(As, Rs)], status
+
+
+def _kappa(m, n, decades, seed):
+    """Singular values over `decades` powers of ten."""
+    rng = np.random.default_rng(seed)
+    U, _ = np.linalg.qr(rng.standard_normal((m, n)))
+    V, _ = np.linalg.qr(rng.standard_normal((n, n)))
+    return (U * np.logspace(0, -decades, n) @ V.T).astype(np.float32)
+
+
+# Panels that are factored twice: near-square matrices, columns of magnitude 1
+# and 1000 in turn, singular values over six decades, a zero column behind the
+# first panel.  A = QR to the rounding of the batch's other tests (1e-6), R
+# within kappa 1e-6 of FP64 LAPACK's, everything finite, the status bit for the
+# zero column only; on the kernel that the built-in table takes and on the wide
+# one.
+@pytest.mark.parametrize("form", ["fp32", "mixed"])
+@pytest.mark.parametrize("pad", [0, 1])
+@pytest.mark.parametrize("variant", [None, WIDE])
+def test_one_projection_second_factor(later, oracle, form, pad, variant):
+    mats = [oracle.gen_uniform(m, n, 17, i) for i, (m, n) in
+            enumerate([(65, 65), (96, 96), (128, 128), (130, 129), (200, 200), (256, 256), (257, 193)])]
+    for m, n in [(1000, 128), (515, 256)]:
+        mats.append((oracle.gen_uniform(m, n, 18, n) * np.where(np.arange(n) % 2, 1000.0, 1.0)).astype(np.float32))
+    mats.append(_kappa(400, 150, 6, 6))
+    dep = oracle.gen_uniform(600, 150, 19, 3)
+    dep[:, 90] = 0.0
+    mats.append(dep)
+    outs, status = _run(later, mats, variant, form, 0, pad)
+    assert list(status) == [0] * (len(mats) - 1) + [1]
+    for i, (A, (Q, R)) in enumerate(zip(mats, outs)):
+        assert np.isfinite(Q).all() and np.isfinite(R).all() and np.array_equal(R, np.triu(R)), (i, A.shape)
+        assert oracle.backward(A, Q, R) < 1e-6, (i, A.shape, oracle.backward(A, Q, R))
+        if i < len(mats) - 1:
+            _, R64 = oracle.lapack_qr64(A)
+            assert oracle.rel_err(R, R64) < 1e-6 * np.linalg.cond(R64) + 1e-6, (i, A.shape)
+    assert np.all(outs[-1][0][:, 90] == 0)
