@@ -8,14 +8,21 @@
 // three sweeps over the rows, 32 at a time, instead of the four that a
 // projection and an update per pass would take:
 //   S1 = Q^T P;    P -= Q S1, S2 = Q^T P;    P -= Q S2, G = P^T P
-// (without reorthogonalisation the middle one is left out), then P = Q_P R_PP
-// by Cholesky QR on G (FP64, chol_dev.h) and one more sweep P <- P R^{-1}.
+// then P = Q_P R_PP by Cholesky QR on G (FP64, chol_dev.h) and one more sweep
+// P <- P R^{-1}.  Without reorthogonalisation P is projected out of Q's
+// 64-column blocks one after another, a block's update and the next one's
+// projection in a sweep:
+//   S1 = Q1^T P;    P -= Q1 S1, S2 = Q2^T P;    ...;    P -= Qb Sb, G = P^T P
+// (block by block the loss of orthogonality grows with kappa 2^-24, all at once
+// with kappa^2 2^-24: 515 x 256 of kappa 1e4 2.2e-3 and 0.32; 1024 matrices of up
+// to 4096 x 256 take 2.75 and 2.51 ms).
 // That is all for a panel whose factor is well conditioned: with an FP64 Gram
 // of FP32 data one Cholesky QR leaves kappa^2 2^-53, far below the rounding of
 // Q's entries to FP32, and what is left of Q in P grows by kappa at most.  When
-// ||R||_F ||R^{-1}||_F (>= kappa, >= w) exceeds 4 w, or a pivot was bad, the
-// normalised panel is projected out of Q once more (with reorthogonalisation)
-// and factored again, so that neither depends on the panel's condition.
+// ||R||_F ||R^{-1}||_F (>= kappa, >= w; the columns' norms are in it) exceeds
+// 4 w, or a pivot was bad, the normalised panel is factored again, after one
+// more projection out of Q where there is reorthogonalisation, so that neither
+// depends on the panel's condition.
 //
 // A chunk of 32 rows of [Q P] is staged in LDS column by column (stride 36:
 // 16-byte reads of 16 columns and 4-byte reads of 16 rows of every fourth
@@ -60,14 +67,18 @@ static_assert(kLds + 1024 <= 163840, "LDS");
 
 typedef float floatx4u __attribute__((ext_vector_type(4), aligned(4)));
 
-// Columns c0 .. c0 + 64 sets - 1 of the matrix, `subs` groups of 32 rows at a
-// time: a chunk fills its four 64-column slots of the buffer whatever the
-// panel's position, so the bytes in flight do not shrink with it.
+// What a sweep reads: K earlier columns Q, the first ku of which it updates with
+// and those from kp on it projects on, and the panel P.
 struct Panel {
-    int m, w, K;          // rows, columns, earlier columns
-    const float *A;       // the matrix: [Q P] are its first K + w columns
+    int m, w;             // rows, columns of P
+    int K, ku, kp;        // multiples of 64
+    const float *Q, *P;
     int64_t lda;
 };
+
+// Columns c0 .. c0 + 64 sets - 1 of [Q P], `subs` groups of 32 rows at a time: a
+// chunk fills its four 64-column slots of the buffer whatever the window's
+// width, so the bytes in flight do not shrink with it.
 
 struct Window {
     int c0, sets, subs;
@@ -108,7 +119,7 @@ template <typename F> __device__ __forceinline__ void for_chunks(const Panel &p,
         const int sub = i / x.sets, c = x.c0 + (t >> 3) + 64 * (i - sub * x.sets);
         rg[i] = kR * min(sub, x.subs - 1) + 4 * (t & 7);
         in[i] = c < nc && sub < x.subs;
-        src[i] = gmem(p.A) + (int64_t)min(c, nc - 1) * p.lda;
+        src[i] = c < p.K ? gmem(p.Q) + (int64_t)c * p.lda : gmem(p.P) + (int64_t)(min(c, nc - 1) - p.K) * p.lda;
     }
     const bool ragged = p.w < kB;
     auto load = [&](Part &part, int i) {
@@ -169,10 +180,11 @@ __device__ __forceinline__ bool gram_tile(int v4, int q, int &x, int &y)
     return q < count;
 }
 
-// One sweep over the rows of [Q P].  update: P -= Q S (S in LDS; P written
-// back); then of the updated rows, project: S' = Q^T P over S, or otherwise
-// G = P^T P to Gs (row stride 65, identity outside w x w).  Wave v: row half
-// v / 4 of a chunk; of the products, Q tiles v % 4 + 4 i against the four tiles
+// One sweep over the rows of [Q P].  update: P -= Q S over Q's first ku columns
+// (S in LDS; P written back); then of the updated rows, project: S' = Q^T P over
+// S, for Q's columns from kp on, or otherwise G = P^T P to Gs (row stride 65,
+// identity outside w x w).  Wave v: row half v / 4 of a chunk; of the products,
+// Q tiles v % 4 + 4 i against the four tiles
 // of P, tile v % 4 of P in the update, the Gram tiles of gram_tile.  (One
 // instance per kind of sweep: with both results' accumulators live, registers
 // spill into the loop, and a reload waits for the loads in flight.)
@@ -183,7 +195,7 @@ __device__ __forceinline__ void sweep(const Panel &p, float *P, char *lds)
     float *S = (float *)lds, *buf = (float *)(lds + kSBytes);
     const int lane = threadIdx.x & 63, v = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int li = lane & 15, g = lane >> 4, v4 = v & 3, h = 16 * (v >> 2);
-    const int K = p.K, qt = K / 64;
+    const int ku = p.ku, kp = p.kp, qt = (p.K - kp) / 64;
     floatx4 acc[kTiles][4];
 #pragma unroll
     for (int i = 0; i < kTiles; ++i)
@@ -198,7 +210,7 @@ __device__ __forceinline__ void sweep(const Panel &p, float *P, char *lds)
         gok[q] = gram_tile(v4, q, gx[q], gy[q]);
     }
     const Window x(p, update || project);
-    const int pc = update || project ? K : 0;  // P's first column in the window
+    const int pc = update || project ? p.K : 0;  // P's first column in the window
     for_chunks(p, x, buf, [&](float *C, int r0, bool full) {
         if (update) {
 #pragma unroll 1
@@ -220,11 +232,11 @@ __device__ __forceinline__ void sweep(const Panel &p, float *P, char *lds)
                 };
                 fetch(sv, qv, 0);
 #pragma unroll 1
-                for (int k = 0; k < K; k += 64) {
+                for (int k = 0; k < ku; k += 64) {
                     fetch(sw, qw, k + 32);
                     d = mfma4(sv[0], qv[0], d);
                     d = mfma4(sv[1], qv[1], d);
-                    fetch(sv, qv, min(k + 64, K - 32));
+                    fetch(sv, qv, min(k + 64, ku - 32));
                     d = mfma4(sw[0], qw[0], d);
                     d = mfma4(sw[1], qw[1], d);
                 }
@@ -256,7 +268,7 @@ __device__ __forceinline__ void sweep(const Panel &p, float *P, char *lds)
 #pragma unroll
                 for (int i = 0; i < kTiles; ++i)
                     if (i < qt) {
-                        const floatx4 a = *(const floatx4 *)(C + x.at(sub, 16 * (v4 + 4 * i) + li) + h + 4 * g);
+                        const floatx4 a = *(const floatx4 *)(C + x.at(sub, kp + 16 * (v4 + 4 * i) + li) + h + 4 * g);
 #pragma unroll
                         for (int u = 0; u < 4; ++u)
 #pragma unroll
@@ -418,53 +430,57 @@ __device__ __forceinline__ void wide_factor(const WgTask &tk, char *lds, bool re
     __shared__ int bad_s;
     bool any_bad = false;
     for (int c0 = 0; c0 < n; c0 += kB) {
+        float *P = tk.A + (int64_t)c0 * tk.lda;
         Panel p;
         p.m = m;
         p.w = min(kB, n - c0);
-        p.K = c0;
-        p.A = tk.A;
+        p.P = P;
         p.lda = tk.lda;
-        float *P = tk.A + (int64_t)c0 * tk.lda;
-        // Step 0: S = Q^T P; 1 (reorth): P -= Q S, S = Q^T P again; 2: P -= Q S
-        // (c0 > 0) and G, factor, apply.  A panel that needs it goes on: 3
-        // (reorth, c0 > 0): S = Q^T P of the normalised panel; 4: as 2 with that
-        // S, and G alone without one (R^{-1} then lies in S's place).
-        int step = c0 > 0 ? 0 : 2;
-        for (;;) {
-            const bool project = step < 2 || step == 3;
-            if (step == 1) sweep<true, true>(p, P, lds);
-            else if (project) sweep<false, true>(p, P, lds);
-            else if (c0 > 0 && (step == 2 || reorth)) sweep<true, false>(p, P, lds);
-            else sweep<false, false>(p, P, lds);  // no S: the first panel, or step 4 without step 3
-            if (project) {
+        const int gw = reorth ? c0 : kB;  // columns of Q in a projection
+        for (int pass = 0;; ++pass) {
+            // Projections of P: twice on all of Q, or once on each block; those
+            // of the normalised panel (pass 1): once on all of Q, or none.
+            const int ng = c0 == 0 ? 0 : reorth ? 2 - pass : pass ? 0 : c0 / kB;
+            for (int g = 0; g < ng; ++g) {
+                const int q0 = reorth ? 0 : kB * g;  // its first column
+                p.kp = reorth || g == 0 ? 0 : kB;
+                p.K = gw + p.kp;
+                p.ku = gw;
+                p.Q = tk.A + (int64_t)(q0 - p.kp) * tk.lda;
+                if (g == 0) sweep<false, true>(p, P, lds);
+                else sweep<true, true>(p, P, lds);
                 // R's rows above the panel: S, + S, + S R1.
-                for (int e = threadIdx.x; e < c0 * p.w; e += kT) {
-                    const int k = e % c0, j = e / c0;
-                    auto *d = R + k + (int64_t)(c0 + j) * ldr;
-                    if (step < 2) {
+                for (int e = threadIdx.x; e < gw * p.w; e += kT) {
+                    const int k = e % gw, j = e / gw;
+                    auto *d = R + q0 + k + (int64_t)(c0 + j) * ldr;
+                    if (pass == 0) {
                         const float s = S[j * kLdS + k];
-                        *d = step ? *d + s : s;
+                        *d = reorth && g ? *d + s : s;
                     } else {
                         double s = 0.0;
                         for (int i = 0; i <= j; ++i) s = fma((double)S[i * kLdS + k], R1[i * kB + j], s);
                         *d = (float)((double)*d + s);
                     }
                 }
-                step += step == 0 && !reorth ? 2 : 1;
-                continue;
             }
+            // The last projection's update (S is still in LDS) and G, or G alone.
+            p.kp = 0;
+            p.K = p.ku = ng ? gw : 0;
+            p.Q = tk.A + (int64_t)(reorth || ng == 0 ? 0 : kB * (ng - 1)) * tk.lda;
+            if (ng) sweep<true, false>(p, P, lds);
+            else sweep<false, false>(p, P, lds);
             const bool bad = factor<kB>(Gs, Rs, Ris, d0, (p.w + 15) / 16);
             if (threadIdx.x == 0) bad_s = bad ? 1 : 0;
             __syncthreads();
             any_bad |= bad_s != 0;
-            const bool again = step == 2 && (bad_s != 0 || !(condition2(Rs, Ris, p.w) <= 16.0 * p.w * p.w));
+            const bool again = pass == 0 && (bad_s != 0 || !(condition2(Rs, Ris, p.w) <= 16.0 * p.w * p.w));
             if (again) {
                 for (int e = threadIdx.x; e < kB * kB; e += kT) R1[e] = Rs[e];
             } else {
                 for (int e = threadIdx.x; e < p.w * p.w; e += kT) {
                     const int i = e % p.w, j = e / p.w;
                     double s = 0.0;
-                    if (step == 2) s = Rs[i * kB + j];
+                    if (pass == 0) s = Rs[i * kB + j];
                     else
                         for (int k = i; k <= j; ++k) s = fma(Rs[i * kB + k], R1[k * kB + j], s);
                     R[c0 + i + (int64_t)(c0 + j) * ldr] = (i <= j) ? (float)s : 0.0f;
@@ -480,7 +496,6 @@ __device__ __forceinline__ void wide_factor(const WgTask &tk, char *lds, bool re
             __syncthreads();
             apply_inverse(p, P, Gs, (float *)(lds + kMat));
             if (!again) break;
-            step = c0 > 0 && reorth ? 3 : 4;
         }
     }
     if (any_bad && threadIdx.x == 0 && tk.status) atomicOr(tk.status, 1);

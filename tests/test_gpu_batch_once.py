@@ -6,7 +6,7 @@ import torch
 
 pytestmark = pytest.mark.gpu
 
-WIDE = 4
+NARROW, WIDE = 1, 4
 
 
 def _run(later, mats, variant, form="fp32", reorth=0, pad=0):
@@ -60,3 +60,19 @@ def test_one_projection_second_factor(later, oracle, form, pad, variant):
             _, R64 = oracle.lapack_qr64(A)
             assert oracle.rel_err(R, R64) < 1e-6 * np.linalg.cond(R64) + 1e-6, (i, A.shape)
     assert np.all(outs[-1][0][:, 90] == 0)
+
+
+# One projection out of 64-column blocks one after another, as on the narrow
+# kernel: the loss of orthogonality grows with kappa, not its square, so it is
+# no worse than twice the narrow kernel's on the same input (other roundings),
+# with the 3e-5 of two projections as the floor.
+@pytest.mark.parametrize("pad", [0, 1])
+def test_one_projection_orthogonality(later, oracle, pad):
+    mats = [oracle.gen_uniform(m, n, 21, i) for i, (m, n) in enumerate([(130, 129), (200, 200), (256, 256), (700, 193)])]
+    mats += [oracle.gen_uniform(m, n, 22, n) + np.float32(3) for m, n in [(300, 256), (400, 200), (1000, 129)]]
+    mats += [_kappa(m, n, d, n + int(d)) for m, n in [(200, 200), (515, 256), (400, 150)] for d in (2, 4, 6)]
+    outs, status = _run(later, mats, WIDE, pad=pad)
+    ref, _ = _run(later, mats, NARROW, pad=pad)
+    assert not status.any()
+    for i, (A, (Q, _), (Qn, _)) in enumerate(zip(mats, outs, ref)):
+        assert oracle.orth(Q) < 2.0 * oracle.orth(Qn) + 3e-5, (i, A.shape, oracle.orth(Q), oracle.orth(Qn))
