@@ -162,10 +162,11 @@ template <typename F> __device__ __forceinline__ void for_chunks(const Panel &p,
     __syncthreads();
 }
 
-__device__ __forceinline__ floatx4 mfma4(floatx4 a, floatx4 b, floatx4 c)
+// Sixteen k, the last of each lane group first.
+__device__ __forceinline__ floatx4 mfma4_down(floatx4 a, floatx4 b, floatx4 c)
 {
 #pragma unroll
-    for (int u = 0; u < 4; ++u) c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[u], b[u], c, 0, 0, 0);
+    for (int u = 3; u >= 0; --u) c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[u], b[u], c, 0, 0, 0);
     return c;
 }
 
@@ -216,7 +217,12 @@ __device__ __forceinline__ void sweep(const Panel &p, float *P, char *lds)
 #pragma unroll 1
             for (int sub = 0; sub < x.subs; ++sub) {
                 // D[n][row] += S[k][n] Q[row][k]: lane n = l % 16 of S, row l % 16
-                // of Q; the operands of the next 32 k are read ahead.
+                // of Q; the operands of the next 32 k are read ahead.  The sum
+                // runs from the last column of Q to the first: where columns
+                // share a direction the first carry the large terms, and the
+                // rest are then added before them, at their own magnitude
+                // (columns with a common mean, 515 x 256: backward error 2.2e-7
+                // in ascending order, 5.8e-8 so; uniform ones the same).
                 const float *sn = S + (16 * v4 + li) * kLdS + 4 * g, *qr = C + x.at(sub, 4 * g) + h + li;
                 float *pr = C + x.at(sub, pc + 16 * v4 + 4 * g) + h + li;
                 floatx4 d = floatx4{0.0f, 0.0f, 0.0f, 0.0f}, sv[2], qv[2], sw[2], qw[2], old;
@@ -230,15 +236,15 @@ __device__ __forceinline__ void sweep(const Panel &p, float *P, char *lds)
                         for (int u = 0; u < 4; ++u) qx[y][u] = qr[(k + 16 * y + u) * kLdC];
                     }
                 };
-                fetch(sv, qv, 0);
+                fetch(sv, qv, ku - 32);
 #pragma unroll 1
-                for (int k = 0; k < ku; k += 64) {
-                    fetch(sw, qw, k + 32);
-                    d = mfma4(sv[0], qv[0], d);
-                    d = mfma4(sv[1], qv[1], d);
-                    fetch(sv, qv, min(k + 64, ku - 32));
-                    d = mfma4(sw[0], qw[0], d);
-                    d = mfma4(sw[1], qw[1], d);
+                for (int k = ku - 64; k >= 0; k -= 64) {
+                    fetch(sw, qw, k);
+                    d = mfma4_down(sv[1], qv[1], d);
+                    d = mfma4_down(sv[0], qv[0], d);
+                    fetch(sv, qv, max(k - 32, 0));
+                    d = mfma4_down(sw[1], qw[1], d);
+                    d = mfma4_down(sw[0], qw[0], d);
                 }
                 const int row = r0 + kR * sub + h + li, col = 16 * v4 + 4 * g;
                 auto *dst = gmem(P) + row + (int64_t)col * p.lda;

@@ -76,3 +76,18 @@ def test_one_projection_orthogonality(later, oracle, pad):
     assert not status.any()
     for i, (A, (Q, _), (Qn, _)) in enumerate(zip(mats, outs, ref)):
         assert oracle.orth(Q) < 2.0 * oracle.orth(Qn) + 3e-5, (i, A.shape, oracle.orth(Q), oracle.orth(Qn))
+
+
+# Columns that share a direction (a common mean): the first columns of Q carry
+# the large terms of an update, and the others' are added before them, so their
+# roundings stay at their own magnitude.  The backward error is within twice the
+# narrow kernel's, which starts each sum from the panel's own entry.
+@pytest.mark.parametrize("reorth", [0, 2])
+def test_correlated_columns_backward(later, oracle, reorth):
+    mats = [oracle.gen_uniform(m, n, 23, n) + np.float32(3) for m, n in [(96, 96), (300, 256), (400, 200), (1000, 129)]]
+    mats += [_kappa(m, n, 6, n) for m, n in [(200, 200), (515, 256)]]
+    outs, status = _run(later, mats, WIDE, reorth=reorth)
+    ref, _ = _run(later, mats, NARROW, reorth=reorth)
+    assert not status.any()
+    for i, (A, (Q, R), (Qn, Rn)) in enumerate(zip(mats, outs, ref)):
+        assert oracle.backward(A, Q, R) < 2.0 * oracle.backward(A, Qn, Rn), (i, A.shape, oracle.backward(A, Q, R))
