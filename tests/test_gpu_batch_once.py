@@ -91,3 +91,18 @@ def test_correlated_columns_backward(later, oracle, reorth):
     assert not status.any()
     for i, (A, (Q, R), (Qn, Rn)) in enumerate(zip(mats, outs, ref)):
         assert oracle.backward(A, Q, R) < 2.0 * oracle.backward(A, Qn, Rn), (i, A.shape, oracle.backward(A, Q, R))
+
+
+# Columns scaled by powers of two scale every sum and product exactly, so Q keeps
+# its bits and R's columns scale exactly, as long as no decision depends on the
+# columns' norms.
+@pytest.mark.parametrize("reorth", [0, 2])
+def test_column_scaling_is_exact(later, oracle, reorth):
+    mats = [oracle.gen_uniform(m, n, 24, i) for i, (m, n) in enumerate([(500, 96), (64, 64), (130, 129), (1000, 256)])]
+    by = [np.where(np.arange(A.shape[1]) % 2, 1024.0, 0.125).astype(np.float32) for A in mats]
+    outs, _ = _run(later, mats, WIDE, reorth=reorth)
+    scaled, status = _run(later, [A * d for A, d in zip(mats, by)], WIDE, reorth=reorth)
+    assert not status.any()
+    for (Q, R), (Qs, Rs), d in zip(outs, scaled, by):
+        assert np.array_equal(Q, Qs) and np.array_equal(R * d, Rs)
+        assert oracle.orth(Qs) < 1e-3
