@@ -21,10 +21,13 @@
 // Q's entries to FP32, and what is left of Q in P grows by kappa at most (kappa
 // of the panel with its columns scaled to norm 1: neither the factor nor a
 // projection depends on their norms).  A panel with a bad pivot or kappa (its
-// Frobenius bound, condition2) above a limit is factored again: 4 w where
+// Frobenius bound, condition2) above a limit is factored again: 2 w where
 // reorthogonalisation has left Q's rounding in P to grow, and then the
 // normalised panel is projected out of Q once more; 2^12 where there is no Q or
-// one projection only, and kappa^2 2^-53 alone counts.  (Unscaled and at 4 w
+// one projection only, and kappa^2 2^-53 alone counts.  (At 4 w a 4000 x 256
+// matrix of kappa 1e3 is left 6.8e-6 from orthogonal, 4.4e-6 on the narrow kernel
+// and 2.3e-6 here; at 1.5 w near-square batches pay, 160 x 160 11% over the narrow
+// kernel.  Unscaled and at 4 w
 // throughout, 512 matrices of 500 x 96 with columns of magnitude 1 and 1000 took
 // 747 us, 420 now; 2048 of 64 x 64 721, 425 now.)
 //
@@ -475,7 +478,7 @@ __device__ __forceinline__ void wide_factor(const WgTask &tk, char *lds, bool re
             if (threadIdx.x == 0) bad_s = bad ? 1 : 0;
             __syncthreads();
             any_bad |= bad_s != 0;
-            const double limit = reorth && c0 > 0 ? 16.0 * p.w * p.w : 0x1p24;
+            const double limit = reorth && c0 > 0 ? 4.0 * p.w * p.w : 0x1p24;
             const bool again = pass == 0 && (bad_s != 0 || !(condition2(Ris, d0, p.w) <= limit));
             if (again) {
                 for (int e = threadIdx.x; e < kB * kB; e += kT) R1[e] = Rs[e];

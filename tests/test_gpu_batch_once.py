@@ -106,3 +106,17 @@ def test_column_scaling_is_exact(later, oracle, reorth):
     for (Q, R), (Qs, Rs), d in zip(outs, scaled, by):
         assert np.array_equal(Q, Qs) and np.array_equal(R * d, Rs)
         assert oracle.orth(Qs) < 1e-3
+
+
+# With two projections what is left of Q in a panel may grow by the panel's
+# condition: panels just under the limit of a second factorisation (singular
+# values of the whole matrix over two and three decades).  Orthogonality within
+# 1.3 times the narrow kernel's, whose panels are half as wide.
+@pytest.mark.parametrize("m,n,decades", [(1000, 128, 2), (515, 256, 3), (4000, 256, 3)])
+def test_two_projections_orthogonality(later, oracle, m, n, decades):
+    mats = [_kappa(m, n, decades, s) for s in (1, 2)]
+    outs, status = _run(later, mats, WIDE, reorth=2)
+    ref, _ = _run(later, mats, NARROW, reorth=2)
+    assert not status.any()
+    for (Q, _), (Qn, _) in zip(outs, ref):
+        assert oracle.orth(Q) < 1.3 * oracle.orth(Qn), (oracle.orth(Q), oracle.orth(Qn))
