@@ -234,9 +234,11 @@ int later_batch_plan_destroy(void *plan);
  * queue, allocating them once with hipMalloc; later_batch_wg_execute
  * enqueues one kernel on `stream` whose workgroups each take whole matrices
  * from the queue (an atomic queue head; the last workgroup to finish resets
- * it, so the plan can be executed again) -- two kernels, one after the
- * other, when the tuning sends a substantial part of the tasks to each of
- * the two kernels below.  Per matrix: left-looking block Gram-Schmidt, each
+ * it, so the plan can be executed again).  When tasks go to both kernels
+ * below, the second is enqueued on a stream of the plan's own that waits for
+ * `stream` and that `stream` then waits for.  A matrix's results depend on
+ * its own size, the options and the tuning only, not on the rest of the
+ * batch.  Per matrix: left-looking block Gram-Schmidt, each
  * panel projected out of all earlier columns of Q twice when opts->reorth
  * != 0 (once otherwise), then factored by Cholesky QR with FP64 Gram
  * matrices; products on MFMA in FP32 (opts->gemm F32 and the split forms),
