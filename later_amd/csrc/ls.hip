@@ -4,6 +4,8 @@
 // blocked back substitution standing in for the reference's recursive TRSM
 // (BLAS/later_rtrsm.cu:75-187): one workgroup per right-hand side keeps the
 // column in LDS in FP64 and works up R in 64-row blocks.
+#include <type_traits>
+
 #include "common.h"
 #include "gemm.h"
 
@@ -66,17 +68,26 @@ __global__ __launch_bounds__(NT) void trsm_upper_kernel(int n, const float *R, i
             double xi = lane < jn ? x[j0 + lane] : 0.0;
 #pragma unroll
             for (int w = 0; w < kWaves; ++w) xi -= part[w][lane];
-            if (!(diag != 0.0f) && lane < jn && status) atomicOr(status, 2);
-            const double inv = diag != 0.0f ? 1.0 / (double)diag : 0.0;
+            // A zero on the diagonal: its unknown is 0, whatever the right-hand
+            // side holds (a product with 0 would keep its sign, or be NaN).
+            const bool zero = !(diag != 0.0f) && lane < jn;
+            if (zero && status) atomicOr(status, 2);
+            const double inv = zero ? 0.0 : 1.0 / (double)diag;
             double res = 0.0;
+            auto solve = [&](auto zeros) {
 #pragma unroll
-            for (int r = TB - 1; r >= 0; --r) {
-                if (r < jn) {
-                    const double xr = readlane_d(xi * inv, r);
-                    res = lane == r ? xr : res;
-                    xi = fma(-(double)d[r], xr, xi);
+                for (int r = TB - 1; r >= 0; --r) {
+                    if (r < jn) {
+                        double t = xi * inv;
+                        if constexpr (decltype(zeros)::value) t = zero ? 0.0 : t;
+                        const double xr = readlane_d(t, r);
+                        res = lane == r ? xr : res;
+                        xi = fma(-(double)d[r], xr, xi);
+                    }
                 }
-            }
+            };
+            if (__builtin_amdgcn_ballot_w64(zero) == 0) solve(std::false_type());
+            else solve(std::true_type());
             if (lane < jn) x[j0 + lane] = res;
         } else if (blk > 0) {
             constexpr int kU = 8;
