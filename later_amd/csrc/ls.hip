@@ -2,8 +2,8 @@
 //
 // Q^T B is the node projection GEMM (gemm.hip).  The triangular solve is a
 // blocked back substitution standing in for the reference's recursive TRSM
-// (BLAS/later_rtrsm.cu:75-187): one workgroup per right-hand side keeps the
-// column in LDS in FP64 and works up R in 64-row blocks.
+// (BLAS/later_rtrsm.cu:75-187): one workgroup per right-hand side, or one wave
+// for several, keeps the columns in LDS in FP64 and works up R in 64-row blocks.
 #include <type_traits>
 
 #include "common.h"
@@ -15,6 +15,35 @@ constexpr int TB = 64;          // diagonal block
 constexpr int kWaves = 8;
 constexpr int NT = 64 * kWaves;
 constexpr int kMaxN = 8192;     // FP64 column in LDS: 64 KiB
+
+// One wave's solve of N right-hand sides with a diagonal block: lane i holds row
+// i (d: its entries right of the diagonal, zeros elsewhere), inv its diagonal's
+// reciprocal and xi its right-hand sides; x_r is read from lane r.
+template <int N>
+__device__ __forceinline__ void solve_block(int jn, const float (&d)[TB], double inv, bool zero, double (&xi)[N],
+                                            double (&res)[N])
+{
+    const int lane = threadIdx.x & 63;
+#pragma unroll
+    for (int c = 0; c < N; ++c) res[c] = 0.0;
+    auto solve = [&](auto zeros) {
+#pragma unroll
+        for (int r = TB - 1; r >= 0; --r) {
+            if (r < jn) {
+#pragma unroll
+                for (int c = 0; c < N; ++c) {
+                    double t = xi[c] * inv;
+                    if constexpr (decltype(zeros)::value) t = zero ? 0.0 : t;
+                    const double xr = readlane_d(t, r);
+                    res[c] = lane == r ? xr : res[c];
+                    xi[c] = fma(-(double)d[r], xr, xi[c]);
+                }
+            }
+        }
+    };
+    if (__builtin_amdgcn_ballot_w64(zero) == 0) solve(std::false_type());
+    else solve(std::true_type());
+}
 
 // Block b's rows need the products with every later block's x.  While wave 0
 // solves block b (lane i owns row i of the diagonal block in registers, x_r is
@@ -73,22 +102,9 @@ __global__ __launch_bounds__(NT) void trsm_upper_kernel(int n, const float *R, i
             const bool zero = !(diag != 0.0f) && lane < jn;
             if (zero && status) atomicOr(status, 2);
             const double inv = zero ? 0.0 : 1.0 / (double)diag;
-            double res = 0.0;
-            auto solve = [&](auto zeros) {
-#pragma unroll
-                for (int r = TB - 1; r >= 0; --r) {
-                    if (r < jn) {
-                        double t = xi * inv;
-                        if constexpr (decltype(zeros)::value) t = zero ? 0.0 : t;
-                        const double xr = readlane_d(t, r);
-                        res = lane == r ? xr : res;
-                        xi = fma(-(double)d[r], xr, xi);
-                    }
-                }
-            };
-            if (__builtin_amdgcn_ballot_w64(zero) == 0) solve(std::false_type());
-            else solve(std::true_type());
-            if (lane < jn) x[j0 + lane] = res;
+            double xs[1] = {xi}, res[1];
+            solve_block(jn, d, inv, zero, xs, res);
+            if (lane < jn) x[j0 + lane] = res[0];
         } else if (blk > 0) {
             constexpr int kU = 8;
             for (int c0 = j0 + jn + wave - 1; c0 < n; c0 += kU * (kWaves - 1)) {
@@ -114,14 +130,107 @@ __global__ __launch_bounds__(NT) void trsm_upper_kernel(int n, const float *R, i
     for (int i = threadIdx.x; i < n; i += NT) b[i] = (float)x[i];
 }
 
+// The same for many right-hand sides: one wave takes N of them and does what
+// the workgroup above does, its waves' sums each in the same order, so that x
+// has the same bits.  Where the CUs are full of right-hand sides the waves that
+// follow a solver only take registers from other solvers (n = 64, 8192 of them:
+// 187 us on the kernel above, 17.5 here).
+template <int N>
+__global__ __launch_bounds__(64) void trsm_upper_many_kernel(int n, int k, const float *R, int64_t ldr, float *B,
+                                                             int64_t ldb, int *status)
+{
+    extern __shared__ __attribute__((aligned(16))) double xs[];  // x of column c at N c .. N c + N - 1
+    constexpr int kStep = kWaves - 1, kShare = TB / kWaves, kU = 4;
+    const int lane = threadIdx.x, k0 = N * blockIdx.x;
+    const int nblk = (n + TB - 1) / TB;
+    for (int i = lane; i < n; i += 64)
+#pragma unroll
+        for (int c = 0; c < N; ++c) xs[N * i + c] = (double)B[(int64_t)min(k0 + c, k - 1) * ldb + i];
+    __syncthreads();
+    double acc[kWaves][N];
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w)
+#pragma unroll
+        for (int c = 0; c < N; ++c) acc[w][c] = 0.0;
+    for (int blk = nblk - 1; blk >= 0; --blk) {
+        const int j0 = blk * TB, jn = min(TB, n - j0);
+        const int row = min(j0 + lane, n - 1), up = j0 - TB + lane;
+        float d[TB];
+#pragma unroll
+        for (int r = 0; r < TB; ++r) d[r] = R[row + (int64_t)min(j0 + r, n - 1) * ldr];
+        const float diag = R[row + (int64_t)row * ldr];
+        double xi[N], res[N];
+#pragma unroll
+        for (int c = 0; c < N; ++c) {
+            xi[c] = lane < jn ? xs[N * row + c] : 0.0;
+#pragma unroll
+            for (int w = 0; w < kWaves; ++w) xi[c] -= acc[w][c];
+        }
+#pragma unroll
+        for (int r = 0; r < TB; ++r) d[r] = lane < r ? d[r] : 0.0f;
+        const bool zero = !(diag != 0.0f) && lane < jn;
+        if (zero && status) atomicOr(status, 2);
+        solve_block(jn, d, zero ? 0.0 : 1.0 / (double)diag, zero, xi, res);
+        if (lane < jn)
+#pragma unroll
+            for (int c = 0; c < N; ++c) xs[N * row + c] = res[c];
+        __syncthreads();
+        if (blk == 0) break;
+        float f[TB];
+#pragma unroll
+        for (int r = 0; r < TB; ++r) f[r] = R[up + (int64_t)(j0 + min(r, jn - 1)) * ldr];
+#pragma unroll
+        for (int w = 0; w < kWaves; ++w)
+#pragma unroll
+            for (int c = 0; c < N; ++c) acc[w][c] = 0.0;
+        for (int c0 = j0 + jn; c0 < n; c0 += kU * kStep) {
+            float v[kU * kStep];
+#pragma unroll
+            for (int u = 0; u < kU * kStep; ++u) v[u] = R[up + (int64_t)min(c0 + u, n - 1) * ldr];
+#pragma unroll
+            for (int u = 0; u < kU * kStep; ++u)
+                if (c0 + u < n)
+#pragma unroll
+                    for (int c = 0; c < N; ++c)
+                        acc[1 + u % kStep][c] = fma((double)v[u], xs[N * (c0 + u) + c], acc[1 + u % kStep][c]);
+        }
+#pragma unroll
+        for (int r = 0; r < TB; ++r)
+            if (r < jn)
+#pragma unroll
+                for (int c = 0; c < N; ++c)
+                    acc[r / kShare][c] = fma((double)f[r], xs[N * (j0 + r) + c], acc[r / kShare][c]);
+    }
+    for (int i = lane; i < n; i += 64)
+#pragma unroll
+        for (int c = 0; c < N; ++c)
+            if (k0 + c < k) B[(int64_t)(k0 + c) * ldb + i] = (float)xs[N * i + c];
+}
+
 } // namespace
 
 int trsm_upper(hipStream_t s, int n, int k, const float *R, int64_t ldr, float *B, int64_t ldb, int *status)
 {
     if (n < 1 || k < 1 || n > kMaxN) return LATER_ERR_SHAPE;
-    // The smaller column array leaves room for several workgroups a CU (servers
-    // solve on several streams at once).
-    if (n <= 1024)
+    // A workgroup a right-hand side while the CUs hold them in a few rounds (one
+    // workgroup a CU: its registers), then one wave for two of them, which takes
+    // 1 to 5 times as long and goes round after 4096 (us, 256 / 512 / 1024 / 2048 right-hand
+    // sides: n = 64 8.8 / 13.9 / 25 / 48 and 9.2 / 9.3 / 9.5 / 9.1; n = 256 22 / 42 / 80 /
+    // 157 and 48 / 50 / 50 / 52; n = 1024 120 / 229 / 457 / 909 and 557 / 559 / 555 / 561), or for
+    // four (16384: n = 64 34 and 30, n = 512 596 and 459, n = 1024 2691 and 2919).  Above
+    // 3072 unknowns the columns' LDS leaves too few waves (n = 4096, 1280: 10.6
+    // and 17.2 ms).
+    const int rounds = (k + 255) / 256;
+    const bool many = n <= 3072 && rounds > (n < 576 ? 1 + n / 192 : 4);
+    if (many && k > 4096 && n <= 512)
+        hipLaunchKernelGGL(trsm_upper_many_kernel<4>, dim3((k + 3) / 4), dim3(64), 4 * n * sizeof(double), s, n, k, R, ldr,
+                           B, ldb, status);
+    else if (many)
+        hipLaunchKernelGGL(trsm_upper_many_kernel<2>, dim3((k + 1) / 2), dim3(64), 2 * n * sizeof(double), s, n, k, R, ldr,
+                           B, ldb, status);
+    // The smaller column array leaves LDS to other streams' kernels (servers
+    // solve on several at once).
+    else if (n <= 1024)
         hipLaunchKernelGGL(trsm_upper_kernel<1024>, dim3(k), dim3(NT), 0, s, n, R, ldr, B, ldb, status);
     else
         hipLaunchKernelGGL(trsm_upper_kernel<kMaxN>, dim3(k), dim3(NT), 0, s, n, R, ldr, B, ldb, status);
