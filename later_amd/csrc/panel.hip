@@ -5,10 +5,14 @@
 // stack is factored recursively, then each block's Q is multiplied by its
 // rows of the stack's Q.  The block kernel is laid out for 64-lane
 // wavefronts instead of the reference's 32x32 thread block of 32-lane warps
-// (QR/panel.cu:246-325): 8 waves, wave v owns columns v, v+8, v+16, v+24 and
-// lane l holds rows l, l+64, ... of them in registers, so the column norm and
-// the projections are single-wave reductions and one barrier per column
-// suffices (the q vector is double-buffered in LDS).
+// (QR/panel.cu:246-325): wave v owns columns 4v .. 4v + 3 and lane l holds rows
+// l, l+64, ... of them in registers, so the column norm and the projections are
+// single-wave reductions, and a finished column passes to the waves behind
+// through LDS with a count, without a barrier.
+//
+// The kernels come for panels of up to 8, 16 and 32 columns (KC): a narrow
+// panel on the widest one keeps waves and registers for columns it does not
+// have (FP64 sums, 1000000 rows: 1 column 59 us, 9 columns 151; 22 and 86 here).
 #include <type_traits>
 
 #include "common.h"
@@ -17,10 +21,8 @@
 
 namespace {
 
-constexpr int kWaves = 8;
-constexpr int kThreads = kWaves * 64;
 constexpr int kCols = 32;                 // max panel width
-constexpr int kCPW = kCols / kWaves;      // columns per wave: wave v owns kCPW v .. kCPW v + kCPW - 1
+constexpr int kCPW = 4;                   // columns per wave: wave v owns kCPW v .. kCPW v + kCPW - 1
 constexpr int kMaxRows = 320;             // rows of a block: 256, or up to 256 + 31 with a merged tail
 
 // sqrt(s) and its reciprocal, both correctly rounded (0 for the reciprocal
@@ -81,12 +83,13 @@ __device__ __forceinline__ bool norm_of(double s, double &nrm, double &inv)
 // 12 us for 256 x 32, where one barrier per column and a column dealt to
 // every eighth wave took 24 us (same bits; FP64 sums 21 and 30 us).
 // RPL: rows per lane, 4 for blocks of up to 256 rows, 5 with a merged tail.
-template <typename Acc, int RPL>
+template <int KC> constexpr int kThreads = 64 * KC / kCPW;
+template <typename Acc, int RPL, int KC>
 __device__ __forceinline__ void mgs_block_body(int m, int w, float *A, int64_t lda, float *Rout, int64_t ldr,
                                                int bh, int nblk, int *status, const int b)
 {
-    __shared__ float qs[kCols][64 * RPL];
-    __shared__ float Rs[kCols][kCols + 1];
+    __shared__ float qs[KC][64 * RPL];
+    __shared__ float Rs[KC][KC + 1];
     __shared__ int published;
 
     const int r0 = b * bh;
@@ -264,37 +267,48 @@ __device__ __forceinline__ void mgs_block_body(int m, int w, float *A, int64_t l
     __syncthreads();
     // R block (w x w, zeros below the diagonal) at rows b*w of Rout.
     auto *Rb = gmem(Rout) + (int64_t)b * w;
-    for (int i = threadIdx.x; i < w * w; i += kThreads) {
+    for (int i = threadIdx.x; i < w * w; i += kThreads<KC>) {
         const int x = i % w, y = i / w;
         Rb[x + (int64_t)y * ldr] = (x <= y) ? Rs[x][y] : 0.0f;
     }
 }
 
-template <typename Acc, int RPL>
-__global__ __launch_bounds__(kThreads) void mgs_block_kernel(int m, int w, float *A, int lda, float *Rout,
-                                                             int ldr, int bh, int nblk, int *status)
+template <typename Acc, int RPL, int KC>
+__global__ __launch_bounds__(kThreads<KC>) void mgs_block_kernel(int m, int w, float *A, int lda, float *Rout,
+                                                                 int ldr, int bh, int nblk, int *status)
 {
-    mgs_block_body<Acc, RPL>(m, w, A, lda, Rout, ldr, bh, nblk, status, blockIdx.x);
+    mgs_block_body<Acc, RPL, KC>(m, w, A, lda, Rout, ldr, bh, nblk, status, blockIdx.x);
 }
 
 template <typename Acc>
-__global__ __launch_bounds__(kThreads) void mgs_block_grouped_kernel(const PanelArgs *args, const int2 *tasks)
+__global__ __launch_bounds__(kThreads<kCols>) void mgs_block_grouped_kernel(const PanelArgs *args, const int2 *tasks)
 {
     const int2 t = tasks[blockIdx.x];
     const PanelArgs a = args[t.x];
-    mgs_block_body<Acc, 5>(a.m, a.w, a.A, a.lda, a.W, a.ldw, kPanelBlockRows, a.nblk, a.status, t.y);
+    mgs_block_body<Acc, 5, kCols>(a.m, a.w, a.A, a.lda, a.W, a.ldw, kPanelBlockRows, a.nblk, a.status, t.y);
+}
+
+// f(columns) with the narrowest of the widths that the kernels come in.
+template <typename F> void by_width(int w, F f)
+{
+    if (w <= 8) f(std::integral_constant<int, 8>());
+    else if (w <= 16) f(std::integral_constant<int, 16>());
+    else f(std::integral_constant<int, kCols>());
 }
 
 // Rows per lane of the largest block: 4 unless a short tail is merged.
 template <typename Acc>
 void launch_mgs(hipStream_t s, int m, int w, float *A, int lda, float *Rout, int ldr, int bh, int nblk, int *status)
 {
-    if (m - (nblk - 1) * bh <= 256)
-        hipLaunchKernelGGL((mgs_block_kernel<Acc, 4>), dim3(nblk), dim3(kThreads), 0, s, m, w, A, lda, Rout, ldr, bh,
-                           nblk, status);
-    else
-        hipLaunchKernelGGL((mgs_block_kernel<Acc, 5>), dim3(nblk), dim3(kThreads), 0, s, m, w, A, lda, Rout, ldr, bh,
-                           nblk, status);
+    by_width(w, [&](auto cols) {
+        constexpr int KC = decltype(cols)::value;
+        if (m - (nblk - 1) * bh <= 256)
+            hipLaunchKernelGGL((mgs_block_kernel<Acc, 4, KC>), dim3(nblk), dim3(kThreads<KC>), 0, s, m, w, A, lda, Rout,
+                               ldr, bh, nblk, status);
+        else
+            hipLaunchKernelGGL((mgs_block_kernel<Acc, 5, KC>), dim3(nblk), dim3(kThreads<KC>), 0, s, m, w, A, lda, Rout,
+                               ldr, bh, nblk, status);
+    });
 }
 
 // A_b <- A_b * W_b for every row block b, W_b = rows b*w .. b*w+w-1 of the
@@ -356,85 +370,95 @@ __global__ __launch_bounds__(256) void tsqr_apply_grouped_kernel(const PanelArgs
 // A's loads are in flight before the first wait: 16384 x 32 takes 7.1 us with
 // the next level's product in it and 4.9 us without, where two launches took
 // 14.5 us each with runtime-strided staging and scalar LDS reads.
-template <typename Acc, int CG, bool FUSED>
+template <typename Acc, int CG, bool FUSED, int KC>
 __global__ __launch_bounds__(256) void tsqr_apply_kernel(int m, int w, float *A, int lda, const float *W, int ldw,
                                                          int nblk, const float *W2, int ldw2, int nblk2)
 {
     constexpr int bh = kPanelBlockRows;
-    __shared__ __attribute__((aligned(16))) Acc Ws[kCols][kCols];  // [j][k]
-    __shared__ float S1[FUSED ? kCols : 1][kCols + 1], S2[FUSED ? 2 : 1][FUSED ? kCols : 1][kCols + 1];
+    __shared__ __attribute__((aligned(16))) Acc Ws[KC][KC];  // [j][k]
+    __shared__ float S1[FUSED ? KC : 1][KC + 1], S2[FUSED ? 2 : 1][FUSED ? KC : 1][KC + 1];
     const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int b = (CG == 4) ? min((int)blockIdx.x * 64 / bh, nblk - 1) : (int)blockIdx.x;
     const int rend = (b == nblk - 1) ? m : (b + 1) * bh;  // rows of the block end here
     const int row0 = (CG == 4) ? (int)blockIdx.x * 64 : b * bh + 64 * wv;
 
-    float v[kCols];
+    float v[KC];
     auto load_rows = [&](int r0) {
         const float *src = A + min(r0 + lane, rend - 1);
 #pragma unroll
-        for (int k = 0; k < kCols; ++k) v[k] = src[(int64_t)min(k, w - 1) * lda];
+        for (int k = 0; k < KC; ++k) v[k] = src[(int64_t)min(k, w - 1) * lda];
     };
     if (CG == 4 || row0 < rend) load_rows(row0);
 
-    const int x = tid & 31;
+    // Thread (x, y0) holds entries (x, y0 + YS u) of the w x w factors (KC = 8:
+    // some hold none).
+    constexpr int YS = 256 / KC, NU = (KC + YS - 1) / YS;
+    const int x = tid & (KC - 1), y0 = tid >> (KC == 8 ? 3 : KC == 16 ? 4 : 5);
     if constexpr (!FUSED) {
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const int y = (tid >> 5) + 8 * u;
+        for (int u = 0; u < NU; ++u) {
+            const int y = y0 + YS * u;
             const float t = W[(int64_t)b * w + min(x, w - 1) + (int64_t)min(y, w - 1) * ldw];
-            Ws[y][x] = (x < w && y < w) ? (Acc)t : (Acc)0;
+            if (KC >= YS || y < KC) Ws[y][x] = (x < w && y < w) ? (Acc)t : (Acc)0;
         }
     } else {
         // Rows g = b w + i of W lie in block min(g / 256, nblk2 - 1) of the
         // next level: one block, or two where w does not divide 256.
         const int b0 = min(b * w / bh, nblk2 - 1), b1 = min((b * w + w - 1) / bh, nblk2 - 1);
-        float t1[4], t2[4], t3[4];
+        float t1[NU], t2[NU], t3[NU];
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const int xc = min(x, w - 1), yc = min((tid >> 5) + 8 * u, w - 1);
+        for (int u = 0; u < NU; ++u) {
+            const int xc = min(x, w - 1), yc = min(y0 + YS * u, w - 1);
             t1[u] = W[(int64_t)b * w + xc + (int64_t)yc * ldw];
             t2[u] = W2[(int64_t)b0 * w + xc + (int64_t)yc * ldw2];
             t3[u] = W2[(int64_t)b1 * w + xc + (int64_t)yc * ldw2];
         }
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const int y = (tid >> 5) + 8 * u;
-            S1[x][y] = t1[u];
-            S2[0][x][y] = t2[u];
-            S2[1][x][y] = t3[u];
+        for (int u = 0; u < NU; ++u) {
+            const int y = y0 + YS * u;
+            if (KC >= YS || y < KC) {
+                S1[x][y] = t1[u];
+                S2[0][x][y] = t2[u];
+                S2[1][x][y] = t3[u];
+            }
         }
         __syncthreads();
         const int sel = (b * w + x) / bh > b0 && b1 > b0 ? 1 : 0;
-        Acc s[4] = {0, 0, 0, 0};
+        Acc s[NU];
+#pragma unroll
+        for (int u = 0; u < NU; ++u) s[u] = (Acc)0;
+        const int yc = KC < YS ? min(y0, KC - 1) : y0;
+#pragma unroll 8
         for (int k = 0; k < w; ++k) {
             const Acc l = (Acc)S1[x][k];
 #pragma unroll
-            for (int u = 0; u < 4; ++u) s[u] = fma(l, (Acc)S2[sel][k][(tid >> 5) + 8 * u], s[u]);
+            for (int u = 0; u < NU; ++u) s[u] = fma(l, (Acc)S2[sel][k][yc + YS * u], s[u]);
         }
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const int y = (tid >> 5) + 8 * u;
-            Ws[y][x] = (x < w && y < w) ? (Acc)(float)s[u] : (Acc)0;
+        for (int u = 0; u < NU; ++u) {
+            const int y = y0 + YS * u;
+            if (KC >= YS || y < KC) Ws[y][x] = (x < w && y < w) ? (Acc)(float)s[u] : (Acc)0;
         }
     }
 #pragma unroll
-    for (int k = 0; k < kCols; ++k)
+    for (int k = 0; k < KC; ++k)
         if (k >= w) v[k] = 0.0f;
     // With CG = 4 this also orders every wave's reads of the tile before any
     // wave's writes to it.
     __syncthreads();
 
-    constexpr int NJ = 4, VW = 16 / sizeof(Acc);  // columns in flight, values of W per LDS read
+    constexpr int PW = KC / CG;  // columns of a wave
+    constexpr int NJ = PW < 4 ? PW : 4, VW = 16 / sizeof(Acc);  // columns in flight, values of W per LDS read
     typedef Acc vec_t __attribute__((ext_vector_type(VW)));
     auto product = [&](int r0) {
         const int row = r0 + lane;
-        const int jbeg = (CG == 4) ? 8 * wv : 0, jend = min(w, (CG == 4) ? 8 * wv + 8 : kCols);
+        const int jbeg = (CG == 4) ? PW * wv : 0, jend = min(w, jbeg + PW);
         for (int j = jbeg; j < jend; j += NJ) {
             Acc s[NJ];
 #pragma unroll
             for (int c = 0; c < NJ; ++c) s[c] = (Acc)0;
 #pragma unroll
-            for (int k = 0; k < kCols; k += VW) {
+            for (int k = 0; k < KC; k += VW) {
                 vec_t wk[NJ];
 #pragma unroll
                 for (int c = 0; c < NJ; ++c) wk[c] = *(const vec_t *)&Ws[j + c][k];
@@ -457,7 +481,7 @@ __global__ __launch_bounds__(256) void tsqr_apply_kernel(int m, int w, float *A,
             if (r0 != row0) {
                 load_rows(r0);
 #pragma unroll
-                for (int k = 0; k < kCols; ++k)
+                for (int k = 0; k < KC; ++k)
                     if (k >= w) v[k] = 0.0f;
             }
             product(r0);
@@ -474,14 +498,16 @@ void launch_apply(hipStream_t s, int m, int w, float *A, int lda, const float *W
     // times finer grid hides the latency of the loads (16384 rows: 7.1 us).
     const bool whole = nblk >= 256;
     const dim3 grid(whole ? nblk : (m + 63) / 64);
-#define LATER_APPLY(CG, F)                                                                                          \
-    hipLaunchKernelGGL((tsqr_apply_kernel<Acc, CG, F>), grid, dim3(256), 0, s, m, w, A, lda, W, ldw, nblk, W2, ldw2, \
-                       nblk2)
-    if (whole && W2) LATER_APPLY(1, true);
-    else if (whole) LATER_APPLY(1, false);
-    else if (W2) LATER_APPLY(4, true);
-    else LATER_APPLY(4, false);
+    by_width(w, [&](auto cols) {
+#define LATER_APPLY(CG, F)                                                                                         \
+    hipLaunchKernelGGL((tsqr_apply_kernel<Acc, CG, F, decltype(cols)::value>), grid, dim3(256), 0, s, m, w, A, lda, W, \
+                       ldw, nblk, W2, ldw2, nblk2)
+        if (whole && W2) LATER_APPLY(1, true);
+        else if (whole) LATER_APPLY(1, false);
+        else if (W2) LATER_APPLY(4, true);
+        else LATER_APPLY(4, false);
 #undef LATER_APPLY
+    });
 }
 
 struct Blocks {
@@ -503,8 +529,8 @@ int panel_blocks(int m, int w) { return plan_blocks(m, w).nblk; }
 int mgs_grouped(hipStream_t s, bool fp64, const PanelArgs *args, const int2 *tasks, int ntasks)
 {
     if (ntasks <= 0) return LATER_OK;
-    if (fp64) hipLaunchKernelGGL(mgs_block_grouped_kernel<double>, dim3(ntasks), dim3(kThreads), 0, s, args, tasks);
-    else hipLaunchKernelGGL(mgs_block_grouped_kernel<float>, dim3(ntasks), dim3(kThreads), 0, s, args, tasks);
+    if (fp64) hipLaunchKernelGGL(mgs_block_grouped_kernel<double>, dim3(ntasks), dim3(kThreads<kCols>), 0, s, args, tasks);
+    else hipLaunchKernelGGL(mgs_block_grouped_kernel<float>, dim3(ntasks), dim3(kThreads<kCols>), 0, s, args, tasks);
     HIP_OK(hipGetLastError());
     return LATER_OK;
 }
