@@ -37,6 +37,7 @@
 #include "chol_dev.h"
 #include "common.h"
 #include "panel.h"
+#include "prof.h"
 
 namespace {
 
@@ -638,15 +639,21 @@ int launch_cholqr(hipStream_t s, int m, int w, float *A, int lda, float *R, int 
     const int nblk = (m + kRows - 1) / kRows;
     // Up to kFusedBlocks blocks every apply workgroup forms the factor itself
     // (the latency of a separate factor launch outweighs the redundancy);
-    // taller panels factor once and apply with more workgroups.
+    // taller panels factor once and apply on the Gram's grid.
     const bool fused = nblk <= kFusedBlocks;
     const dim3 rgrid((Shape<W>::P + 31) / 32);
     int n = 0;
-    if (up)
+    if (up) {
+        // Timed with the other updates, by the update's own work (its time
+        // holds the Gram's).
+        const int tok = prof_start(s);
         hipLaunchKernelGGL(chol_update_gram_kernel<W>, dim3(G), dim3(kThreads), 0, s, m, w, A, (int64_t)lda, work, up->k,
                            up->Q, up->ldq, up->C, up->ldc);
-    else
+        prof_stop(tok, s, PROF_GEMM_UPDATE, 2.0 * m * w * up->k,
+                  4.0 * ((double)m * up->k + 2.0 * m * w + (double)up->k * w));
+    } else {
         hipLaunchKernelGGL(chol_gram_kernel<W>, dim3(G), dim3(kThreads), 0, s, m, w, (const float *)A, (int64_t)lda, work);
+    }
     ++n;
     if (G > kDirect) {
         hipLaunchKernelGGL(chol_reduce_kernel<W>, rgrid, dim3(256), 0, s, cw.p1, G, w, cw.g);

@@ -9,7 +9,7 @@
 // node updates, the R2 R1 composition and the first pass's projections of
 // enough tiles; PROF_PROJ_I8: the int8 four-slice projections (the mixed
 // form's second pass); PROF_GEMM_UPDATE and PROF_GEMM_PROJ hold the other
-// products.
+// products, the updates that also form a leaf's first Gram among them.
 enum { PROF_GEMM_PROJ = 0, PROF_GEMM_UPDATE = 1, PROF_PANEL = 2, PROF_OTHER = 3, PROF_UPDATE_X3 = 4,
        PROF_PROJ_I8 = 5, PROF_NCLASS = 6 };
 
