@@ -21,6 +21,7 @@ struct GemmArgs {
     int update;                    // 0: C = result; 1: C += alpha * result (FP32); 2: the same in FP64
     float alpha;
     int tri;                       // op(A), B upper triangular: skip zero tiles and K ranges
+    int tested;                    // fused conversion: bounds-tested loads throughout (same results)
     // Pre-split operands (nullptr: convert A and B in the kernel): 16-bit
     // pieces, K-major (row i of op(A) at Ah + i * ldah, piece c at
     // Ah + c * psa), already scaled by 2^a_exp / 2^b_exp[j].

@@ -651,7 +651,7 @@ __device__ __forceinline__ void gemm_body(const GemmArgs &g, const int tm, const
     // tile row take the tested loads.
     int it0 = 0;
     if constexpr (!PRE) {
-        const int nin = (AKM || m0 + BM <= g.M) ? (kend - kbeg) / BK : 0;  // slabs with every k inside
+        const int nin = !g.tested && (AKM || m0 + BM <= g.M) ? (kend - kbeg) / BK : 0;  // slabs with every k inside
         auto load_inside = [&](int slot_it, SA &a, SB &b) {
             a.load_inside(g.A, g.lda, m0, g.M, kbeg + slot_it * BK);
             b.load_inside(g.B, g.ldb, n0, g.N, kbeg + slot_it * BK);
@@ -1809,6 +1809,24 @@ int64_t gemm_proj_work_floats(int m, int n1, int n2, int chunk)
     return ns > 1 ? (int64_t)ns * n1 * n2 * (chunk > 0 ? 2 : 1) : 0;
 }
 
+// Projections whose operands are several times the 256 MB cache and whose
+// products are cheap (one 16-bit piece, or two) keep the tested loads: with the
+// rings' lead the tiles that share rows drift apart, and the rows are fetched
+// again (us, ring / tested: FP16 262144 x 1024 x 1024 4030 / 2490, 131072 x 1024 x 1024
+// 1190 / 1050, 262144 x 512 x 512 669 / 620, but 131072 x 512 x 512 269 / 290 and 65536 x
+// 2048 x 2048 1195 / 1216; hi/lo 262144 x 1024 x 1024 4054 / 3748, 131072 x 1024 x 1024
+// 1776 / 1830; three pieces and FP32 are ahead on the ring throughout).  Unaligned
+// operands stay on the ring: tested, they are read value by value (262145 x 512 x
+// 512 814 / 1543).
+static bool tested_loads(int prec, int64_t m, int64_t n1, int64_t n2, const float *Q, int64_t ldq, const float *B,
+                         int64_t ldb)
+{
+    const int64_t bytes = 4 * m * (n1 + n2);
+    const bool aligned = ((ldq | ldb) & 3) == 0 && (((uintptr_t)Q | (uintptr_t)B) & 15) == 0;
+    return aligned && (prec == GEMM_F16 || prec == GEMM_BF16 ? bytes > 1000000000
+                                                             : prec == GEMM_F16X3 && bytes > 2000000000);
+}
+
 static void set_pieces(GemmArgs &g, const Pieces *ah, const Pieces *bh)
 {
     const bool pre = ah && bh && ah->p && bh->p;
@@ -1845,6 +1863,7 @@ int gemm_proj(hipStream_t s, int prec, int m, int n1, int n2, const float *Q, in
     g.update = 0;
     g.alpha = 1.0f;
     g.tri = 0;
+    g.tested = tested_loads(prec, m, n1, n2, Q, ldq, B, ldb);
     set_pieces(g, qh, bh);
     if (i8) {
         // Byte operands counted in pairs of bytes (K padded to 64 rows);
@@ -1897,6 +1916,7 @@ int gemm_nn(hipStream_t s, int prec, int M, int N, int K, float alpha, const flo
             int *launches, const Pieces *ah, const Pieces *bh)
 {
     GemmArgs g;
+    g.tested = 0;
     g.M = M; g.N = N; g.K = K;
     g.A = A; g.lda = lda; g.B = B; g.ldb = ldb; g.C = C; g.ldc = ldc;
     g.a_exp = a_exp; g.b_exp = b_exp;
