@@ -19,8 +19,8 @@ constexpr int kMaxN = 8192;     // FP64 column in LDS: 64 KiB
 // One wave's solve of N right-hand sides with a diagonal block: lane i holds row
 // i (d: its entries right of the diagonal, zeros elsewhere), inv its diagonal's
 // reciprocal and xi its right-hand sides; x_r is read from lane r.
-template <int N>
-__device__ __forceinline__ void solve_block(int jn, const float (&d)[TB], double inv, bool zero, double (&xi)[N],
+template <int N, int T>
+__device__ __forceinline__ void solve_block(int jn, const float (&d)[T], double inv, bool zero, double (&xi)[N],
                                             double (&res)[N])
 {
     const int lane = threadIdx.x & 63;
@@ -28,7 +28,7 @@ __device__ __forceinline__ void solve_block(int jn, const float (&d)[TB], double
     for (int c = 0; c < N; ++c) res[c] = 0.0;
     auto solve = [&](auto zeros) {
 #pragma unroll
-        for (int r = TB - 1; r >= 0; --r) {
+        for (int r = T - 1; r >= 0; --r) {
             if (r < jn) {
 #pragma unroll
                 for (int c = 0; c < N; ++c) {
@@ -134,15 +134,16 @@ __global__ __launch_bounds__(NT) void trsm_upper_kernel(int n, const float *R, i
 // the workgroup above does, its waves' sums each in the same order, so that x
 // has the same bits.  Where the CUs are full of right-hand sides the waves that
 // follow a solver only take registers from other solvers (n = 64, 8192 of them:
-// 187 us on the kernel above, 17.5 here).
-template <int N>
+// 187 us on the kernel above, 17.5 here).  T: rows of a diagonal block, 16 for
+// systems that one such block holds.
+template <int N, int T>
 __global__ __launch_bounds__(64) void trsm_upper_many_kernel(int n, int k, const float *R, int64_t ldr, float *B,
                                                              int64_t ldb, int *status)
 {
     extern __shared__ __attribute__((aligned(16))) double xs[];  // x of column c at N c .. N c + N - 1
-    constexpr int kStep = kWaves - 1, kShare = TB / kWaves, kU = 4;
+    constexpr int kStep = kWaves - 1, kShare = T / kWaves, kU = 4;
     const int lane = threadIdx.x, k0 = N * blockIdx.x;
-    const int nblk = (n + TB - 1) / TB;
+    const int nblk = (n + T - 1) / T;
     for (int i = lane; i < n; i += 64)
 #pragma unroll
         for (int c = 0; c < N; ++c) xs[N * i + c] = (double)B[(int64_t)min(k0 + c, k - 1) * ldb + i];
@@ -153,11 +154,11 @@ __global__ __launch_bounds__(64) void trsm_upper_many_kernel(int n, int k, const
 #pragma unroll
         for (int c = 0; c < N; ++c) acc[w][c] = 0.0;
     for (int blk = nblk - 1; blk >= 0; --blk) {
-        const int j0 = blk * TB, jn = min(TB, n - j0);
-        const int row = min(j0 + lane, n - 1), up = j0 - TB + lane;
-        float d[TB];
+        const int j0 = blk * T, jn = min(T, n - j0);
+        const int row = min(j0 + lane, n - 1), up = j0 - T + lane;
+        float d[T];
 #pragma unroll
-        for (int r = 0; r < TB; ++r) d[r] = R[row + (int64_t)min(j0 + r, n - 1) * ldr];
+        for (int r = 0; r < T; ++r) d[r] = R[row + (int64_t)min(j0 + r, n - 1) * ldr];
         const float diag = R[row + (int64_t)row * ldr];
         double xi[N], res[N];
 #pragma unroll
@@ -167,7 +168,7 @@ __global__ __launch_bounds__(64) void trsm_upper_many_kernel(int n, int k, const
             for (int w = 0; w < kWaves; ++w) xi[c] -= acc[w][c];
         }
 #pragma unroll
-        for (int r = 0; r < TB; ++r) d[r] = lane < r ? d[r] : 0.0f;
+        for (int r = 0; r < T; ++r) d[r] = lane < r ? d[r] : 0.0f;
         const bool zero = !(diag != 0.0f) && lane < jn;
         if (zero && status) atomicOr(status, 2);
         solve_block(jn, d, zero ? 0.0 : 1.0 / (double)diag, zero, xi, res);
@@ -176,9 +177,9 @@ __global__ __launch_bounds__(64) void trsm_upper_many_kernel(int n, int k, const
             for (int c = 0; c < N; ++c) xs[N * row + c] = res[c];
         __syncthreads();
         if (blk == 0) break;
-        float f[TB];
+        float f[T];
 #pragma unroll
-        for (int r = 0; r < TB; ++r) f[r] = R[up + (int64_t)(j0 + min(r, jn - 1)) * ldr];
+        for (int r = 0; r < T; ++r) f[r] = R[up + (int64_t)(j0 + min(r, jn - 1)) * ldr];
 #pragma unroll
         for (int w = 0; w < kWaves; ++w)
 #pragma unroll
@@ -195,7 +196,7 @@ __global__ __launch_bounds__(64) void trsm_upper_many_kernel(int n, int k, const
                         acc[1 + u % kStep][c] = fma((double)v[u], xs[N * (c0 + u) + c], acc[1 + u % kStep][c]);
         }
 #pragma unroll
-        for (int r = 0; r < TB; ++r)
+        for (int r = 0; r < T; ++r)
             if (r < jn)
 #pragma unroll
                 for (int c = 0; c < N; ++c)
@@ -212,6 +213,10 @@ __global__ __launch_bounds__(64) void trsm_upper_many_kernel(int n, int k, const
 int trsm_upper(hipStream_t s, int n, int k, const float *R, int64_t ldr, float *B, int64_t ldb, int *status)
 {
     if (n < 1 || k < 1 || n > kMaxN) return LATER_ERR_SHAPE;
+    // Up to 16 unknowns a block of 16 rows holds them all: a fixed cost of 2.6 us
+    // where blocks of 64 rows have 5.7 (8 unknowns, 1 right-hand side; 1000 of them
+    // 3.6 and 6.6, 20000 7.7 and 19).
+    //
     // A workgroup a right-hand side while the CUs hold them in a few rounds (one
     // workgroup a CU: its registers), then one wave for two of them, which takes
     // 1 to 5 times as long and goes round after 4096 (us, 256 / 512 / 1024 / 2048 right-hand
@@ -222,11 +227,17 @@ int trsm_upper(hipStream_t s, int n, int k, const float *R, int64_t ldr, float *
     // and 17.2 ms).
     const int rounds = (k + 255) / 256;
     const bool many = n <= 3072 && rounds > (n < 576 ? 1 + n / 192 : 4);
-    if (many && k > 4096 && n <= 512)
-        hipLaunchKernelGGL(trsm_upper_many_kernel<4>, dim3((k + 3) / 4), dim3(64), 4 * n * sizeof(double), s, n, k, R, ldr,
+    if (n <= 16 && k <= 4096)
+        hipLaunchKernelGGL((trsm_upper_many_kernel<1, 16>), dim3(k), dim3(64), n * sizeof(double), s, n, k, R, ldr, B, ldb,
+                           status);
+    else if (n <= 16)
+        hipLaunchKernelGGL((trsm_upper_many_kernel<4, 16>), dim3((k + 3) / 4), dim3(64), 4 * n * sizeof(double), s, n, k, R,
+                           ldr, B, ldb, status);
+    else if (many && k > 4096 && n <= 512)
+        hipLaunchKernelGGL((trsm_upper_many_kernel<4, TB>), dim3((k + 3) / 4), dim3(64), 4 * n * sizeof(double), s, n, k, R, ldr,
                            B, ldb, status);
     else if (many)
-        hipLaunchKernelGGL(trsm_upper_many_kernel<2>, dim3((k + 1) / 2), dim3(64), 2 * n * sizeof(double), s, n, k, R, ldr,
+        hipLaunchKernelGGL((trsm_upper_many_kernel<2, TB>), dim3((k + 1) / 2), dim3(64), 2 * n * sizeof(double), s, n, k, R, ldr,
                            B, ldb, status);
     // The smaller column array leaves LDS to other streams' kernels (servers
     // solve on several at once).

@@ -20,7 +20,7 @@ def _system(oracle, n, k, seed=31):
 # The unknown of a zero on the diagonal is +0 whatever its right-hand side holds
 # (negative, infinite, NaN), and the rows above are solved with that 0: their
 # residual is within 2^-24 (plus n FP64 roundings) of |R| |x|.
-@pytest.mark.parametrize("n", [1, 40, 64, 65, 200])
+@pytest.mark.parametrize("n", [1, 16, 17, 40, 64, 65, 200])
 @pytest.mark.parametrize("value", [-1.0, np.inf, -np.inf, np.nan])
 def test_zero_diagonal_unknown_is_zero(later, oracle, n, value):
     R, B = _system(oracle, n, 3)
@@ -42,7 +42,7 @@ def test_zero_diagonal_unknown_is_zero(later, oracle, n, value):
 # Every right-hand side gets the same bits however many there are: a workgroup
 # each, a wave for two and a wave for four, at the edges of their ranges, with
 # zeros on the diagonal and a partly filled last wave.
-@pytest.mark.parametrize("n", [1, 8, 63, 64, 65, 130, 256, 512, 513, 600])
+@pytest.mark.parametrize("n", [1, 8, 16, 17, 63, 64, 65, 130, 256, 512, 513, 600])
 @pytest.mark.parametrize("k", [513, 1537, 4097])
 @pytest.mark.parametrize("zero", [False, True])
 def test_same_bits_for_many_right_hand_sides(later, oracle, n, k, zero):
