@@ -228,31 +228,31 @@ int later_batch_plan_execute(void *plan, void *stream);
 int later_batch_plan_launches(void *plan);
 int later_batch_plan_destroy(void *plan);
 
-/* Batched QR in ONE persistent launch (no counterpart in the reference).
- * later_batch_wg_create builds the task table (one task per matrix, ordered
- * by size bucket and decreasing cost, largest first) and the device work
- * queue, allocating them once with hipMalloc; later_batch_wg_execute
- * enqueues one kernel on `stream` whose workgroups each take whole matrices
- * from the queue (an atomic queue head; the last workgroup to finish resets
- * it, so the plan can be executed again).  When tasks go to both kernels
- * below, the second is enqueued on a stream of the plan's own that waits for
- * `stream` and that `stream` then waits for.  A matrix's results depend on
- * its own size, the options and the tuning only, not on the rest of the
- * batch.  Per matrix: left-looking block Gram-Schmidt, each
- * panel projected out of all earlier columns of Q twice when opts->reorth
- * != 0 (once otherwise), then factored by Cholesky QR with FP64 Gram
- * matrices; products on MFMA in FP32 (opts->gemm F32 and the split forms),
- * BF16 or FP16 (opts->gemm BF16 / F16).  A is overwritten by Q and R (n x n,
- * zero below the diagonal).  status (optional, count ints): bit 0 set for a
- * matrix whose panel had a bad pivot.  tuning (optional):
- * LATER_BATCH_BUCKETS variant ids, one per size bucket
+/* Batched QR in one persistent launch, or two side by side (no counterpart in
+ * the reference).  later_batch_wg_create builds the task table (one task per
+ * matrix, ordered by size bucket and decreasing cost, largest first) and the
+ * device work queue, allocating them once with hipMalloc;
+ * later_batch_wg_execute enqueues one kernel on `stream` whose workgroups each
+ * take whole matrices from the queue (an atomic queue head; the last workgroup
+ * to finish resets it, so the plan can be executed again).  When tasks go to
+ * both kernels below, the second is enqueued on a stream of the plan's own
+ * that waits for `stream` and that `stream` then waits for.  A matrix's
+ * results depend on its own size, the options and the tuning only, not on the
+ * rest of the batch.
+ *   Per matrix: left-looking block Gram-Schmidt, each panel projected out of
+ * all earlier columns of Q twice when opts->reorth != 0 (once otherwise), then
+ * factored by Cholesky QR with FP64 Gram matrices; products on MFMA in FP32
+ * (opts->gemm F32 and the split forms), BF16 or FP16 (opts->gemm BF16 / F16).
+ * A is overwritten by Q and R (n x n, zero below the diagonal).  status
+ * (optional, count ints): bit 0 set for a matrix whose panel had a bad pivot.
+ *   tuning (optional): LATER_BATCH_BUCKETS variant ids, one per size bucket
  * later_batch_wg_bucket(m, n) = 7 (min(ceil(n/32), 8) - 1) +
  * clamp(floor(log2 m) - 6, 0, 6); variants v = 0 .. 3 use 16 << (v & 1)
  * columns per panel and blocks of 64 << (v >> 1) earlier Q columns, variant
- * 4 is the wide kernel (64-column panels, all earlier columns at once; FP32
- * products, 4 <= m, n <= 256, other tasks take the table's best of 0 .. 3);
- * NULL (or -1 entries) selects the built-in table written by
- * later_amd/autotune.py. */
+ * 4 is the wide kernel (64-column panels, all earlier columns at once, or in
+ * blocks of 64 when they are projected out once; FP32 products, 4 <= m,
+ * n <= 256, other tasks take the table's best of 0 .. 3); NULL (or -1 entries)
+ * selects the built-in table written by later_amd/autotune.py. */
 #define LATER_BATCH_BUCKETS 56
 int later_batch_wg_create(int count, const int *m, const int *n, float *const *A, const int *lda,
                           float *const *R, const int *ldr, int *status, const later_opts *opts,

@@ -1,8 +1,8 @@
-// Batched QR in one persistent launch: every workgroup takes whole matrices
-// from a device work queue and factors each one by itself.  This file holds
-// the queue, the plan and the kernel for 16-bit products, narrow matrices and
-// more than 256 columns; FP32 products of 33 .. 256 columns run
-// batch_wide.hip's.
+// Batched QR in one persistent launch (two side by side when a batch holds
+// tasks of both kernels): every workgroup takes whole matrices from a device
+// work queue and factors each one by itself.  This file holds the queue, the
+// plan and the kernel for 16-bit products, narrow matrices and more than 256
+// columns; FP32 products of 33 .. 256 columns run batch_wide.hip's.
 //
 // The queue is the task table, ordered by size bucket and, inside a bucket,
 // by decreasing cost (largest matrices first, so the long tasks start

@@ -27,9 +27,8 @@
 // one projection only, and kappa^2 2^-53 alone counts.  (At 4 w a 4000 x 256
 // matrix of kappa 1e3 is left 6.8e-6 from orthogonal, 4.4e-6 on the narrow kernel
 // and 2.3e-6 here; at 1.5 w near-square batches pay, 160 x 160 11% over the narrow
-// kernel.  Unscaled and at 4 w
-// throughout, 512 matrices of 500 x 96 with columns of magnitude 1 and 1000 took
-// 747 us, 420 now; 2048 of 64 x 64 721, 425 now.)
+// kernel.  Unscaled and at 4 w throughout, 512 matrices of 500 x 96 with columns
+// of magnitude 1 and 1000 took 755 us, 420 now; 2048 of 64 x 64 722, 425 now.)
 //
 // A chunk of 32 rows of [Q P] is staged in LDS column by column (stride 36:
 // 16-byte reads of 16 columns and 4-byte reads of 16 rows of every fourth
@@ -40,8 +39,8 @@
 // Bound: the matrix cores of one CU (FP32 4 m n^2 at 614 GFLOP/s, FP64 Gram and
 // apply at 258; 57% busy on a 4096 x 256 matrix, the rest the barriers between
 // the phases of a chunk), and the largest matrix of a batch on its workgroup:
-// 4096 x 256 takes 3.4 ms, 9.3 on the narrow kernel; 1024 matrices of up to
-// that size 3.8 ms, 9.8 there.
+// 4096 x 256 takes 3.45 ms, 9.3 on the narrow kernel; 1024 matrices of up to
+// that size 3.7 ms, 9.9 there.
 #include <type_traits>
 
 #include "batch_wg.h"

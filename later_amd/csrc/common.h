@@ -38,12 +38,6 @@ __device__ __forceinline__ int dpp_i(int v)
 }
 
 template <int CTRL, int ROWS = 0xF>
-__device__ __forceinline__ float dpp_f(float v)
-{
-    return __int_as_float(dpp_i<CTRL, ROWS>(__float_as_int(v)));
-}
-
-template <int CTRL, int ROWS = 0xF>
 __device__ __forceinline__ double dpp_d(double v)
 {
     const int lo = dpp_i<CTRL, ROWS>(__double2loint(v));
