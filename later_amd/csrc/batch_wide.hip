@@ -15,7 +15,7 @@
 //   S1 = Q1^T P;    P -= Q1 S1, S2 = Q2^T P;    ...;    P -= Qb Sb, G = P^T P
 // (block by block the loss of orthogonality grows with kappa 2^-24, all at once
 // with kappa^2 2^-24: 515 x 256 of kappa 1e4 2.2e-3 and 0.32; 1024 matrices of up
-// to 4096 x 256 take 2.75 and 2.51 ms).
+// to 4096 x 256 take 2.57 and 2.51 ms).
 // That is all for a panel whose factor is well conditioned: with an FP64 Gram
 // of FP32 data one Cholesky QR leaves kappa^2 2^-53, far below the rounding of
 // Q's entries to FP32, and what is left of Q in P grows by kappa at most (kappa
@@ -419,7 +419,9 @@ __device__ __forceinline__ double condition2(const double *Ris, const double *d0
     return s * w / kPivotRel;
 }
 
-__device__ __forceinline__ void wide_factor(const WgTask &tk, char *lds, bool reorth)
+// (An instance with reorthogonalisation and one without: one for both spills
+// more, 1024 matrices 3.70 ms for 3.65, and 2.80 for 2.57 without.)
+template <bool reorth> __device__ __forceinline__ void wide_factor(const WgTask &tk, char *lds)
 {
     const int m = tk.m, n = tk.n;
     const int64_t ldr = tk.ldr;
@@ -506,7 +508,7 @@ __device__ __forceinline__ void wide_factor(const WgTask &tk, char *lds, bool re
     if (any_bad && threadIdx.x == 0 && tk.status) atomicOr(tk.status, 1);
 }
 
-__global__ __launch_bounds__(kT) void batch_wide_kernel(const WgTask *tasks, int ntasks, WgQueue *q, int reorth)
+template <bool reorth> __global__ __launch_bounds__(kT) void batch_wide_kernel(const WgTask *tasks, int ntasks, WgQueue *q)
 {
     __shared__ __attribute__((aligned(16))) char lds[kLds];
     for (;;) {
@@ -515,7 +517,7 @@ __global__ __launch_bounds__(kT) void batch_wide_kernel(const WgTask *tasks, int
         const WgTask tk = tasks[t];
         if (threadIdx.x == 0 && tk.status) *tk.status = 0;
         __syncthreads();
-        wide_factor(tk, lds, reorth != 0);
+        wide_factor<reorth>(tk, lds);
         __syncthreads();
     }
     wg_leave(q);
@@ -525,7 +527,8 @@ __global__ __launch_bounds__(kT) void batch_wide_kernel(const WgTask *tasks, int
 
 int batch_wide_launch(hipStream_t s, const WgTask *tasks, int ntasks, WgQueue *q, int grid, bool reorth)
 {
-    hipLaunchKernelGGL(batch_wide_kernel, dim3(grid), dim3(kT), 0, s, tasks, ntasks, q, reorth ? 1 : 0);
+    if (reorth) hipLaunchKernelGGL(batch_wide_kernel<true>, dim3(grid), dim3(kT), 0, s, tasks, ntasks, q);
+    else hipLaunchKernelGGL(batch_wide_kernel<false>, dim3(grid), dim3(kT), 0, s, tasks, ntasks, q);
     HIP_OK(hipGetLastError());
     return LATER_OK;
 }
