@@ -595,10 +595,10 @@ struct WgPlan {
 
     ~WgPlan()
     {
+        if (dev) hipFree(dev);  // first: it waits for launches that are still running
         if (fork) hipEventDestroy(fork);
         if (join) hipEventDestroy(join);
         if (side) hipStreamDestroy(side);
-        if (dev) hipFree(dev);
     }
 };
 

@@ -80,3 +80,18 @@ def test_stream_order_and_capture(later):
         torch.cuda.synchronize()
         assert _equal(want, [(a.cpu().numpy(), r.cpu().numpy()) for a, r in got]), rep
     plan.close()
+
+
+# A plan may be closed behind its last launch: what was enqueued still runs, and
+# later work on the stream follows it.
+def test_close_behind_a_launch(later):
+    src, As, Rs = _inputs(later)
+    plan = later.BatchWg(As, Rs, later.opts("mixed"))
+    want = _run(plan, src, As, Rs)
+    for a, s in zip(As, src):
+        a.copy_(s)
+    plan.execute()
+    plan.close()
+    got = [(a.clone(), r.clone()) for a, r in zip(As, Rs)]
+    torch.cuda.synchronize()
+    assert _equal(want, [(a.cpu().numpy(), r.cpu().numpy()) for a, r in got])
